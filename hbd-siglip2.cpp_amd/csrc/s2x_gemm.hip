@@ -44,16 +44,23 @@
 // W scales are fp16 bits transposed, dT[kb * ldT + n].
 //
 // LDS layout of one stage (bytes):
-//   XQ  [KS][128 rows][32]  X quants, the two 16-byte chunks of row r at
-//                            chunk position c ^ swz(r)
-//   WQ  [KS][128 rows][32]  W quants, same swizzle
+//   XQ  [128 rows][KS][32]  X quants, a row's KS blocks together, 16-byte
+//                            chunk c (of 8) of row r at position c ^ swz8(r)
+//   WQ  [128 rows][KS][32]  W quants, same swizzle
 //   XS  [128][KS] u32        X ds words, a row's KS blocks together (as in
 //                            the ds plane: one 16-byte DMA lane per row)
 //   WS  [KS][128] u16        W scales in the dT plane's column order
 //                            (columns j and j + 32 of each 64-column half
 //                            in one 32-bit word)
-// A fragment read (lane l: row l & 31, chunk l >> 5, 16 bytes) then touches
-// 16 distinct 16-byte bank groups per 16 lanes: no bank conflicts.
+// A fragment read of block j (lane l: row l & 31, chunk 2 j + (l >> 5), 16
+// bytes) touches distinct 16-byte bank groups in every 8 and every 16
+// consecutive lanes: no bank conflicts.  A quant DMA instruction brings the
+// 128 bytes (4 blocks) of 8 rows, 8 cache lines (16 where rows are no whole
+// lines apart), not 32 bytes of 32 rows: the vector memory path handles an
+// instruction line by line (1 KB as 8 whole lines takes it 15 to 17 cycles,
+// as 32 quarter lines 30, measured alone).  It is what the few-rows forms
+// wait for: M = 729 fc2 23.3 -> 20.8 us, M = 64 fc2 21.6 -> 17.7; at M =
+// 23,328, where the matrix pipe and the VALU bound the loop, 1 to 3 %.
 #include "s2x_device.h"
 #include "s2x_kernels.h"
 
@@ -83,8 +90,8 @@ struct Cfg {
     static constexpr bool LAT = LAT_;
     // waves of 32 TM x 32 TN outputs, WN of them along N
     static constexpr int WN = BN / (32 * TN), NWAVE = BM / (32 * TM) * WN, NT = NWAVE * WAVE;
-    static constexpr int XQ = 0;                  // [KS][BM][32] X quants
-    static constexpr int WQ = XQ + KS * BM * 32;  // [KS][BN][32] W quants
+    static constexpr int XQ = 0;                  // [BM][KS][32] X quants
+    static constexpr int WQ = XQ + KS * BM * 32;  // [BN][KS][32] W quants
     // [XS_ROWS][KS] u32 X ds words: at least 64 rows, the rows one X-scale
     // DMA instruction writes (rows past a 32-row tile are never read)
     static constexpr int XS_ROWS = BM < 64 ? 64 : BM;
@@ -95,17 +102,18 @@ struct Cfg {
     static constexpr int WG_PER_CU = 2 * LDS_BYTES <= 163840 ? 2 : 1;
     static constexpr int WPE = LAT ? 2 : WG_PER_CU * NWAVE / 4;  // waves per SIMD
     // DMA instructions per stage: QPX X-quant and QPW W-quant per wave (each
-    // 32 rows of one block: KS BM / 32 and 4 KS per stage); the scales, 16
+    // 8 rows of the stage's KS blocks: BM / 8 and 16 per stage); the scales, 16
     // bytes per lane (a row's 4 consecutive ds words, or 8 W scales of one
     // block), by the first NSX + 1 waves: waves 0 .. NSX - 1 the X scales
     // of 64 rows each, wave NSX the W scales.  The issue cost of these
     // instructions, not their bytes, is what the K loop feels, hence the
     // scales in as few of them as their 16-byte rows allow.
     static constexpr int NSX = BM < 64 ? 1 : BM / 64;
-    static constexpr int QPX = KS * (BM / 32) / NWAVE, QPW = KS * (BN / 32) / NWAVE;
+    static constexpr int QPX = BM / 8 / NWAVE, QPW = BN / 8 / NWAVE;
     static_assert(KS == 4, "stage of 4 blocks: one 16-byte ds row per X row");
     static_assert(BM == 128 || BM == 64 || (BM == 32 && LAT && TN == 1), "tile rows");
-    static_assert(QPX >= 1 && QPW >= 1 && QPX <= KS && QPW <= KS, "DMA split");
+    static_assert(QPX >= 1 && QPW >= 1 && QPX * NWAVE * 8 == BM && QPW * NWAVE * 8 == BN, "DMA split");
+    static_assert(STAGE % 128 == 0 && WQ % 128 == 0, "quant rows: chunk positions by xor");
     static_assert(NS == 2 || (LAT && NS <= 4), "ring: two stages, or up to four in the latency form");
     static_assert(NSX + 1 <= NWAVE, "scale DMA waves");
     static_assert(LDS_BYTES * WG_PER_CU <= 163840, "LDS");
@@ -124,8 +132,10 @@ __device__ __forceinline__ void static_for(F &&f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// chunk permutation of the two 16-byte chunks of a 32-byte row
-__device__ __forceinline__ int swz(int r) { return ((r >> 2) ^ (r >> 3)) & 1; }
+// chunk permutation of the eight 16-byte chunks of a 128-byte row: rows r of
+// any 8 consecutive ones, and the even (odd) rows of any aligned 16, have
+// distinct swz8, so the same chunk of those rows lies in distinct bank groups
+__device__ __forceinline__ int swz8(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
                                       uint8_t *lds_wave_base) {
@@ -530,18 +540,25 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 
     // Per-lane DMA source offsets (relative to the tile's first row / column;
     // the K position goes into the scalar offset).
-    //   X quants, instructions t < QPX: i = QPX wave + t, block i % KS, rows
-    //             32 (i / KS) .. + 31 (= 32 (QPX wave / KS) for every t)
+    //   X quants, instructions t < QPX: rows 8 (QPX wave + t) .. + 7, the
+    //             stage's 4 blocks (128 bytes: 8 lanes) of each
     //   W quants, instructions t < QPW: likewise with QPW
     //   X scales: waves w < NSX, rows 64 w + lane, the ds words of blocks
     //             k0 .. k0 + 3 (16 bytes)
     //   W scales: wave NSX, block lane / 16, columns 8 (lane % 16) .. + 7
-    uint32_t vqx, vqw, vxs, vws;
+    uint32_t vqx[C::QPX], vqw[C::QPW], vxs, vws;
     {
-        const int rx = 32 * (C::QPX * wave / KS) + (lane >> 1);
-        vqx = (uint32_t)(rx * row_bytes) + (uint32_t)(((lane & 1) ^ swz(rx)) * 16);
-        const int rw = 32 * (C::QPW * wave / KS) + (lane >> 1);
-        vqw = (uint32_t)(rw * row_bytes) + (uint32_t)(((lane & 1) ^ swz(rw)) * 16);
+        // chunk at position p of row r: p ^ swz8(r); in a GEMM of fewer than
+        // KS blocks (one stage) the chunks of the missing blocks are out of
+        // range
+        const auto quant_off = [&](int r) {
+            const int c = (lane & 7) ^ swz8(r);
+            return c < 2 * KB ? (uint32_t)(r * row_bytes) + (uint32_t)(c * 16) : OOB_OFF;
+        };
+#pragma unroll
+        for (int t = 0; t < C::QPX; ++t) vqx[t] = quant_off(8 * (C::QPX * wave + t) + (lane >> 3));
+#pragma unroll
+        for (int t = 0; t < C::QPW; ++t) vqw[t] = quant_off(8 * (C::QPW * wave + t) + (lane >> 3));
         vxs = (uint32_t)((min(wave, C::NSX - 1) * 64 + lane) * ld_ds * 4);
         vws = (uint32_t)((lane >> 4) * ldT * 2 + (lane & 15) * 16);
     }
@@ -569,8 +586,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // kpos(g) = KB - KS, so its block kb0 + j lands in slot j + shift of the
     // stage buffer (shift = kb0 - kpos); a GEMM of fewer than KS blocks has
     // one partial stage, fetched by the first issue (outside the K loop)
-    // with a zero-size buffer per missing block and out-of-range lanes for
-    // the missing scales.  ROLE (a constant per wave: 1 X scales, 2 W
+    // with out-of-range lanes for the missing blocks and scales.  ROLE (a constant per wave: 1 X scales, 2 W
     // scales, 0 neither) is a template value, so that no branch splits the
     // K loop.
     // PART: 0 the X quants, 1 the W quants, 2 the scales, -1 all three
@@ -583,15 +599,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             if (KB < KS) {
                 // the only stage, blocks 0 .. KB - 1 of KS
 #pragma unroll
-                for (int t = 0; t < C::QPX; ++t) {
-                    const int i = C::QPX * wave + t, j = i % KS;
-                    dma16(j < KB ? xr_live : none, vqx, j * 32, sb + XQ + j * BM * 32 + (i / KS) * 1024);
-                }
+                for (int t = 0; t < C::QPX; ++t) dma16(xr_live, vqx[t], 0, sb + XQ + (C::QPX * wave + t) * 1024);
 #pragma unroll
-                for (int t = 0; t < C::QPW; ++t) {
-                    const int i = C::QPW * wave + t, j = i % KS;
-                    dma16(j < KB ? wr_live : none, vqw, j * 32, sb + WQ + j * BN * 32 + (i / KS) * 1024);
-                }
+                for (int t = 0; t < C::QPW; ++t) dma16(wr_live, vqw[t], 0, sb + WQ + (C::QPW * wave + t) * 1024);
                 if constexpr (ROLE == 1) {
                     // one 4-byte DMA per ds word: 16 rows x KS words per
                     // instruction, the words of missing blocks out of range
@@ -612,17 +622,11 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         const uint32_t k0 = (uint32_t)kpos(g);
         if constexpr (PART == 0 || PART < 0) {
 #pragma unroll
-            for (int t = 0; t < C::QPX; ++t) {
-                const int i = C::QPX * wave + t, j = i % KS;
-                dma16(xr, vqx, (k0 + j) * 32, sb + XQ + j * BM * 32 + (i / KS) * 1024);
-            }
+            for (int t = 0; t < C::QPX; ++t) dma16(xr, vqx[t], k0 * 32, sb + XQ + (C::QPX * wave + t) * 1024);
         }
         if constexpr (PART == 1 || PART < 0) {
 #pragma unroll
-            for (int t = 0; t < C::QPW; ++t) {
-                const int i = C::QPW * wave + t, j = i % KS;
-                dma16(wr, vqw, (k0 + j) * 32, sb + WQ + j * BN * 32 + (i / KS) * 1024);
-            }
+            for (int t = 0; t < C::QPW; ++t) dma16(wr, vqw[t], k0 * 32, sb + WQ + (C::QPW * wave + t) * 1024);
         }
         if constexpr (PART == 2 || PART < 0) {
             if constexpr (ROLE == 1)
@@ -643,8 +647,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 
     // fragment addresses (bytes within a stage buffer) of this lane
     const int xrow = wm * 32 * TM + lr, wcol = wn * 32 * TN + lr;
-    const int a_off = XQ + xrow * 32 + ((lh ^ swz(lr)) * 16);
-    const int b_off = WQ + wcol * 32 + ((lh ^ swz(lr)) * 16);
+    // (block 0's; block j's chunks 2 j + lh sit at the offset ^ 32 j)
+    const int a_off = XQ + xrow * 128 + ((lh ^ swz8(lr)) * 16);
+    const int b_off = WQ + wcol * 128 + ((lh ^ swz8(lr)) * 16);
     const int sx_off = XS + xrow * 16;
     // the 32-bit word of W scales (column j | column j + 32 << 16 of a
     // 64-column group) holding this lane's columns, and the low half of the
@@ -658,10 +663,10 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     auto load_frag = [&](const uint8_t *sb, int j, Frag<TM, TN> &f) {
 #pragma unroll
         for (int a = 0; a < TM; ++a)
-            f.a[a] = *reinterpret_cast<const v4i *>(sb + a_off + j * BM * 32 + a * 32 * 32);
+            f.a[a] = *reinterpret_cast<const v4i *>(sb + (a_off ^ (j * 32)) + a * 32 * 128);
 #pragma unroll
         for (int b = 0; b < TN; ++b)
-            f.b[b] = *reinterpret_cast<const v4i *>(sb + b_off + j * BN * 32 + b * 32 * 32);
+            f.b[b] = *reinterpret_cast<const v4i *>(sb + (b_off ^ (j * 32)) + b * 32 * 128);
 #pragma unroll
         for (int a = 0; a < TM; ++a) f.xw[a] = *reinterpret_cast<const uint32_t *>(sb + sx_off + j * 4 + a * 32 * 16);
         f.wp = *reinterpret_cast<const uint32_t *>(sb + sw_off + j * BN * 2);
