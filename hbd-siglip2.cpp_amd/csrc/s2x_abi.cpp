@@ -80,7 +80,7 @@ int s2x_quantize_q8_1(const float *x, int64_t K, int64_t M, int64_t ldx, int64_t
 // ---------------------------------------------------------------------------
 size_t s2x_weight_bytes(int64_t K_pad, int64_t N) {
     if (K_pad <= 0 || N <= 0 || K_pad % QK_ != 0) return 0;
-    return weight_planes_bytes(K_pad, N);
+    return weight_planes_bytes(K_pad, N, K_pad);
 }
 
 int s2x_weight_create_in(const void *raw_dev, int64_t K_pad, int64_t N, void *dev_buf,
@@ -96,7 +96,7 @@ int s2x_weight_create_in(const void *raw_dev, int64_t K_pad, int64_t N, void *de
     s2x_weight *w = new s2x_weight();
     w->mem = dev_buf;
     w->owns = false;
-    w->view = planes_view(dev_buf, K_pad, N);
+    w->view = planes_view(dev_buf, K_pad, N, K_pad);
     hipError_t e = repack_into(raw_dev, w->view, (hipStream_t)stream);
     if (e != hipSuccess) {
         delete w;
@@ -257,7 +257,7 @@ int s2x_mul_mat_q8_0_f32(const void *w_raw, int64_t K_pad, int64_t N, const floa
         return fail(S2X_ERR_INVALID_ARG, "mul_mat_q8_0_f32: misaligned pointer");
     uint8_t *ws = (uint8_t *)workspace;
     hipStream_t s = (hipStream_t)stream;
-    const WeightView wv = planes_view(ws + L.w_off, K_pad, N);
+    const WeightView wv = planes_view(ws + L.w_off, K_pad, N, K_pad);
     hipError_t e = repack_into(w_raw, wv, s);
     if (e != hipSuccess) return hip_fail(e, "repack launch");
     Q81Out o;

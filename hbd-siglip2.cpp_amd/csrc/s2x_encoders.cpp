@@ -54,14 +54,14 @@ int weight_upload(const void *raw, bool is_host, int64_t K_pad, int64_t N, hipSt
         src = tmp;
     }
     void *planes = nullptr;
-    if (hipMalloc(&planes, weight_planes_bytes(K_pad, N)) != hipSuccess) {
+    if (hipMalloc(&planes, weight_planes_bytes(K_pad, N, gemm_ld_q(K_pad))) != hipSuccess) {
         if (tmp) (void)hipFree(tmp);
         return fail(S2X_ERR_OOM, "weight upload: hipMalloc planes failed");
     }
     s2x_weight *w = new s2x_weight();
     w->mem = planes;
     w->owns = true;
-    w->view = planes_view(planes, K_pad, N);
+    w->view = planes_view(planes, K_pad, N, gemm_ld_q(K_pad));
     hipError_t e = repack_into(src, w->view, stream);
     if (e == hipSuccess && tmp) e = hipStreamSynchronize(stream);
     if (tmp) (void)hipFree(tmp);
@@ -349,12 +349,13 @@ struct Tower {
             b = timing.get();
             S2X_HIP_TRY(hipEventRecord(a, stream));
         }
+        const int64_t ldx = from_qs2 ? ld_q2(M) : 0;
         const int ns = splits(w->view.K_pad / QK_, e);
         const hipError_t err =
             ns > 1 ? launch_gemm_split_k(w->view, xq.as<int8_t>(), xd.as<uint32_t>(),
-                                         w->view.K_pad / QK_, M, y, ldy, e, ns, part.as<float>(), stream)
+                                         w->view.K_pad / QK_, M, y, ldy, e, ns, part.as<float>(), stream, ldx)
                    : launch_gemm(w->view, xq.as<int8_t>(), xd.as<uint32_t>(), w->view.K_pad / QK_,
-                                 M, y, ldy, e, stream);
+                                 M, y, ldy, e, stream, ldx);
         if (err != hipSuccess) return hip_fail(err, "gemm launch");
         if (timing.on) {
             S2X_HIP_TRY(hipEventRecord(b, stream));
@@ -362,6 +363,10 @@ struct Tower {
         }
         return S2X_OK;
     }
+
+    // Row stride of fc2's Q8_1 input: whole cache lines for the tiled GEMMs;
+    // the few-row form (at most 8 rows) takes rows back to back
+    int64_t ld_q2(int64_t M) const { return M <= 8 ? F_pad : gemm_ld_q(F_pad); }
 
     // The MLP of a block or of the MAP head on M rows whose LN2 + Q8_1 is in
     // qs / ds: fc1 (+bias, GELU, and Q8_1 -- or f16 for an F16 ffn_down --
@@ -383,6 +388,7 @@ struct Tower {
         ep.q_ds = ds2.as<uint32_t>();
         ep.q_kpad = F_pad;
         ep.q_ldds = F_pad / QK_;
+        ep.q_ld = ld_q2(M);
         S2X_TRY(gemm(up, M, nullptr, 0, ep, H));
         return gemm(down.q8, M, y, H, EpiParams{EPI_BIAS_RESID, down_b, resid, H, 0, 0}, F, true);
     }
@@ -417,7 +423,7 @@ struct Tower {
         if (down_f16) {
             S2X_TRY(ensure(h16, sizeof(_Float16) * (size_t)(M * F_pad), stream));
         } else {
-            S2X_TRY(ensure(qs2, (size_t)(M * F_pad), stream));
+            S2X_TRY(ensure(qs2, (size_t)(M * gemm_ld_q(F_pad)), stream));
             S2X_TRY(ensure(ds2, sizeof(uint32_t) * (size_t)(M * (F_pad / QK_)), stream));
         }
         S2X_TRY(ensure(att, sizeof(float) * (size_t)(M * H), stream));

@@ -248,7 +248,7 @@ __device__ __forceinline__ void epilogue(float (&acc)[TM][TN][16], float scale, 
                 qs += dpp_i<0xb1>(qs);
                 const int m = mw + a * 32 + row;
                 if (m < M) {
-                    const int64_t off = (int64_t)m * epi.q_kpad + nb0 + half * 16;
+                    const int64_t off = (int64_t)m * epi.q_ld + nb0 + half * 16;
                     *reinterpret_cast<uint4 *>(epi.q_out8 + off) =
                         make_uint4(pack4_i8(qi[0], qi[1], qi[2], qi[3]), pack4_i8(qi[4], qi[5], qi[6], qi[7]),
                                    pack4_i8(qi[8], qi[9], qi[10], qi[11]),
@@ -511,8 +511,8 @@ __device__ __forceinline__ void epilogue(float (&acc)[TM][TN][16], float scale, 
 
 template <class C, int EPI>
 __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE))) void k_gemm(
-    const uint8_t *__restrict__ xq, const uint32_t *__restrict__ xds, int64_t ld_ds,
-    const uint8_t *__restrict__ wq, const uint16_t *__restrict__ wdT, int64_t ldT, int M, int N,
+    const uint8_t *__restrict__ xq, int64_t ldx, const uint32_t *__restrict__ xds, int64_t ld_ds,
+    const uint8_t *__restrict__ wq, int64_t ldw, const uint16_t *__restrict__ wdT, int64_t ldT, int M, int N,
     int KB, float *__restrict__ y, int64_t ldy, EpiParams epi) {
     constexpr int BM = C::BM, NS = C::NS, KS = C::KS, STAGE = C::STAGE, TM = C::TM;
     constexpr int XQ = C::XQ, WQ = C::WQ, XS = C::XS, WS = C::WS;
@@ -528,7 +528,6 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     tile_of(xcd_linear(blockIdx.x, gridDim.x), m_tiles, n_tiles, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     const int KB_all = KB;
-    const int64_t row_bytes = (int64_t)KB_all * QK;  // X and W rows: all KB blocks
     // a K split: this workgroup's blocks kbs .. kbs + KB - 1 (EPI_NONE)
     int kbs = 0;
     if (EPI == EPI_NONE && epi.kb_split > 0) {
@@ -551,24 +550,24 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         // chunk at position p of row r: p ^ swz8(r); in a GEMM of fewer than
         // KS blocks (one stage) the chunks of the missing blocks are out of
         // range
-        const auto quant_off = [&](int r) {
+        const auto quant_off = [&](int r, int64_t ld) {
             const int c = (lane & 7) ^ swz8(r);
-            return c < 2 * KB ? (uint32_t)(r * row_bytes) + (uint32_t)(c * 16) : OOB_OFF;
+            return c < 2 * KB ? (uint32_t)(r * ld) + (uint32_t)(c * 16) : OOB_OFF;
         };
 #pragma unroll
-        for (int t = 0; t < C::QPX; ++t) vqx[t] = quant_off(8 * (C::QPX * wave + t) + (lane >> 3));
+        for (int t = 0; t < C::QPX; ++t) vqx[t] = quant_off(8 * (C::QPX * wave + t) + (lane >> 3), ldx);
 #pragma unroll
-        for (int t = 0; t < C::QPW; ++t) vqw[t] = quant_off(8 * (C::QPW * wave + t) + (lane >> 3));
+        for (int t = 0; t < C::QPW; ++t) vqw[t] = quant_off(8 * (C::QPW * wave + t) + (lane >> 3), ldw);
         vxs = (uint32_t)((min(wave, C::NSX - 1) * 64 + lane) * ld_ds * 4);
         vws = (uint32_t)((lane >> 4) * ldT * 2 + (lane & 15) * 16);
     }
     // (the bases start at block kbs; the ranges end where the planes end)
     const __amdgpu_buffer_rsrc_t xr_live = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(xq + (int64_t)m0 * row_bytes + kbs * QK), (short)0,
-        clip32((int64_t)(M - m0) * row_bytes - kbs * QK), BUF_DW3);
+        (void *)(xq + (int64_t)m0 * ldx + kbs * QK), (short)0,
+        clip32((int64_t)(M - m0) * ldx - kbs * QK), BUF_DW3);
     const __amdgpu_buffer_rsrc_t wr_live = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(wq + (int64_t)n0 * row_bytes + kbs * QK), (short)0,
-        clip32((int64_t)(N - n0) * row_bytes - kbs * QK), BUF_DW3);
+        (void *)(wq + (int64_t)n0 * ldw + kbs * QK), (short)0,
+        clip32((int64_t)(N - n0) * ldw - kbs * QK), BUF_DW3);
     const __amdgpu_buffer_rsrc_t xsr_live = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(xds + (int64_t)m0 * ld_ds + kbs), (short)0,
         clip32((int64_t)(M - m0) * ld_ds * 4 - kbs * 4), BUF_DW3);
@@ -952,7 +951,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 }
 
 template <class C, int EPI>
-hipError_t run(const WeightView &w, const int8_t *xq, const uint32_t *xds, int64_t ld_ds,
+hipError_t run(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds, int64_t ld_ds,
                int64_t M, float *y, int64_t ldy, const EpiParams &epi, hipStream_t stream) {
     auto kern = k_gemm<C, EPI>;
     static bool attr_set = false;  // idempotent; a racing second call repeats it harmlessly
@@ -969,9 +968,9 @@ hipError_t run(const WeightView &w, const int8_t *xq, const uint32_t *xds, int64
     // without scales (the block-dot dump) the scale DMA reads a zero-size
     // buffer at a valid address
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles, splits), dim3(C::NT), C::LDS_BYTES, stream,
-                       reinterpret_cast<const uint8_t *>(xq),
+                       reinterpret_cast<const uint8_t *>(xq), ldx,
                        xds ? xds : reinterpret_cast<const uint32_t *>(xq), xds ? ld_ds : 0,
-                       reinterpret_cast<const uint8_t *>(w.qs), w.dT, w.ldT, (int)M, (int)w.N,
+                       reinterpret_cast<const uint8_t *>(w.qs), w.ld_qs, w.dT, w.ldT, (int)M, (int)w.N,
                        (int)(w.K_pad / QK), y, ldy, epi);
     return hipGetLastError();
 }
@@ -1159,7 +1158,7 @@ __global__ __launch_bounds__(256) void k_split_sum(const float *__restrict__ par
 hipError_t launch_gemm_split_k(const WeightView &w, const int8_t *xq, const uint32_t *xds,
                                int64_t ld_ds, int64_t M, float *y, int64_t ldy,
                                const EpiParams &epi, int n_split, float *part,
-                               hipStream_t stream) {
+                               hipStream_t stream, int64_t ldx) {
     if (M == 0 || w.N == 0) return hipSuccess;
     const int64_t KB = w.K_pad / QK;
     const bool resid = epi.kind == EPI_BIAS_RESID;
@@ -1173,7 +1172,7 @@ hipError_t launch_gemm_split_k(const WeightView &w, const int8_t *xq, const uint
     e.kind = EPI_NONE;
     e.kb_split = (int)per;
     e.y_split = M * w.N;
-    hipError_t err = launch_gemm(w, xq, xds, ld_ds, M, part, w.N, e, stream);
+    hipError_t err = launch_gemm(w, xq, xds, ld_ds, M, part, w.N, e, stream, ldx);
     if (err != hipSuccess) return err;
     const bool vec = w.N % 4 == 0 && ldy % 4 == 0 && (!resid || epi.ld_resid % 4 == 0);
     const int64_t n = M * (vec ? w.N / 4 : w.N);
@@ -1222,7 +1221,7 @@ static int64_t gv_lds_bytes(int64_t M, int64_t K_pad) {
 template <int CW, int EPI>
 __global__ __launch_bounds__(GV_NT) void k_gemv(const int8_t *__restrict__ xq,
                                                 const uint32_t *__restrict__ xds, int64_t ld_ds,
-                                                const int8_t *__restrict__ wq,
+                                                const int8_t *__restrict__ wq, int64_t ldw,
                                                 const uint16_t *__restrict__ wdT, int64_t ldT,
                                                 int K_pad, int M, int N, float *__restrict__ y,
                                                 int64_t ldy, EpiParams epi) {
@@ -1243,7 +1242,7 @@ __global__ __launch_bounds__(GV_NT) void k_gemv(const int8_t *__restrict__ xq,
         const int i = tid + j * GV_NT, c = i / KB, kb = i - c * KB;
         wv[j][0] = wv[j][1] = int4{0, 0, 0, 0};
         if (i < CW * KB && n0 + c < N) {
-            const int4 *p = reinterpret_cast<const int4 *>(wq + (int64_t)(n0 + c) * K_pad + kb * QK);
+            const int4 *p = reinterpret_cast<const int4 *>(wq + (int64_t)(n0 + c) * ldw + kb * QK);
             wv[j][0] = p[0];
             wv[j][1] = p[1];
         }
@@ -1333,7 +1332,7 @@ __global__ __launch_bounds__(GV_NT) void k_gemv(const int8_t *__restrict__ xq,
             const float d = a / 127.0f;
             const float inv = a != 0.0f ? 127.0f / a : 0.0f;
             int s = 0;
-            uint32_t *qo = reinterpret_cast<uint32_t *>(epi.q_out8 + (int64_t)tid * epi.q_kpad + n0);
+            uint32_t *qo = reinterpret_cast<uint32_t *>(epi.q_out8 + (int64_t)tid * epi.q_ld + n0);
             for (int k = 0; k < 32; k += 4) {
                 const int q0 = q8_round(v[k], inv), q1 = q8_round(v[k + 1], inv);
                 const int q2 = q8_round(v[k + 2], inv), q3 = q8_round(v[k + 3], inv);
@@ -1359,7 +1358,7 @@ static hipError_t run_gemv(const WeightView &w, const int8_t *xq, const uint32_t
     }
     const int64_t cols = EPI == EPI_GELU_Q81 ? epi.q_kpad : w.N;
     hipLaunchKernelGGL(kern, dim3((unsigned)((cols + CW - 1) / CW)), dim3(GV_NT),
-                       (unsigned)gv_lds_bytes<CW>(M, w.K_pad), stream, xq, xds, ld_ds, w.qs, w.dT,
+                       (unsigned)gv_lds_bytes<CW>(M, w.K_pad), stream, xq, xds, ld_ds, w.qs, w.ld_qs, w.dT,
                        w.ldT, (int)w.K_pad, (int)M, (int)w.N, y, ldy, epi);
     return hipGetLastError();
 }
@@ -1373,7 +1372,8 @@ static bool gv_fits(int64_t M, const WeightView &w) {
     return M <= GV_MAX_M && CW * KB <= GV_IT * GV_NT && M * KB <= GV_IT * GV_NT &&
            M * (w.K_pad / 16) <= GV_XIT * GV_NT && gv_lds_bytes<CW>(M, w.K_pad) <= GV_LDS_MAX;
 }
-static bool use_gemv(int64_t M, const WeightView &w, const EpiParams &epi) {
+static bool use_gemv(int64_t M, int64_t ldx, const WeightView &w, const EpiParams &epi) {
+    if (ldx != w.K_pad) return false;  // (its X rows lie back to back)
     switch (epi.kind) {
     case EPI_NONE: return epi.kb_split == 0 && gv_fits<8>(M, w);
     case EPI_BIAS:
@@ -1421,8 +1421,9 @@ using Small4T = gemm::Cfg<4, 4, 32, true, 1, 1>;
 using Small3 = gemm::Cfg<4, 3, 64, true>;
 
 template <int E>
-static hipError_t run_small(const WeightView &w, const int8_t *xq, const uint32_t *xds, int64_t ld_ds,
-                            int64_t M, float *y, int64_t ldy, const EpiParams &epi, hipStream_t stream);
+static hipError_t run_small(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds,
+                            int64_t ld_ds, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
+                            hipStream_t stream);
 
 static bool use_small(int64_t M, int64_t N) {
     return ((M + 127) / 128) * ((N + 127) / 128) < 2 * 256;
@@ -1431,22 +1432,26 @@ static bool small_ring4(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 1
 static bool small_rows32(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 127) / 128) < 256; }
 
 hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xds, int64_t ld_ds,
-                       int64_t M, float *y, int64_t ldy, const EpiParams &epi,
-                       hipStream_t stream) {
+                       int64_t M, float *y, int64_t ldy, const EpiParams &epi_in,
+                       hipStream_t stream, int64_t ldx) {
     using C = Wide;
     if (M == 0 || w.N == 0) return hipSuccess;
+    EpiParams epi = epi_in;
+    if (epi.q_ld == 0) epi.q_ld = epi.q_kpad;
+    if (ldx == 0) ldx = w.K_pad;
     const int64_t KB = w.K_pad / QK;
     if (!w.qs || !w.dT || !xq || w.K_pad <= 0 || w.K_pad % QK || w.ldT < (w.N + 127) / 128 * 128 ||
         M > (1 << 30) || w.N > (1 << 30) || ((uintptr_t)xq & 15) || ((uintptr_t)w.qs & 15) ||
         ((uintptr_t)xds & 3) || (epi.kind != EPI_DUMP_I && (!xds || ld_ds < KB)) ||
-        (int64_t)C::BM * KB * QK > 0x7fffffff || w.ldT * KB * 2 > 0x7fffffff ||
+        ldx < w.K_pad || ldx % 16 || w.ld_qs < w.K_pad || w.ld_qs % 16 || (int64_t)C::BM * ldx > 0x7fffffff ||
+        (int64_t)gemm::BN * w.ld_qs > 0x7fffffff || w.ldT * KB * 2 > 0x7fffffff ||
         C::BM * ld_ds * 4 > 0x7fffffff || C::BM * ldy * 4 > 0x7fffffff ||
         (epi.kb_split != 0 && (epi.kind != EPI_NONE || epi.kb_split < 0 || epi.y_split < M * ldy)))
         return hipErrorInvalidValue;
 #define S2X_RUN(E)                                                                     \
-    (use_gemv(M, w, epi) ? run_gemv_epi<E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream)  \
-     : !use_small(M, w.N) ? gemm::run<C, E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream) \
-                          : run_small<E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream))
+    (use_gemv(M, ldx, w, epi) ? run_gemv_epi<E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream)  \
+     : !use_small(M, w.N) ? gemm::run<C, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream) \
+                          : run_small<E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream))
     switch (epi.kind) {
     case EPI_NONE: return S2X_RUN(EPI_NONE);
     case EPI_BIAS: return S2X_RUN(EPI_BIAS);
@@ -1461,7 +1466,7 @@ hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xd
         return S2X_RUN(EPI_DUMP_I);
     case EPI_GELU_Q81:
         if (!epi.q_out8 || !epi.q_ds || !epi.bias || epi.q_kpad % QK || epi.q_kpad < w.N ||
-            epi.q_kpad - w.N >= QK || epi.q_ldds < epi.q_kpad / QK ||
+            epi.q_kpad - w.N >= QK || epi.q_ldds < epi.q_kpad / QK || epi.q_ld < epi.q_kpad || epi.q_ld % 16 ||
             ((uintptr_t)epi.q_out8 & 15) || ((uintptr_t)epi.q_ds & 3))
             return hipErrorInvalidValue;
         return S2X_RUN(EPI_GELU_Q81);
@@ -1481,16 +1486,17 @@ hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xd
 }
 
 template <int E>
-static hipError_t run_small(const WeightView &w, const int8_t *xq, const uint32_t *xds, int64_t ld_ds,
-                            int64_t M, float *y, int64_t ldy, const EpiParams &epi, hipStream_t stream) {
+static hipError_t run_small(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds,
+                            int64_t ld_ds, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
+                            hipStream_t stream) {
     constexpr bool plain = E == EPI_NONE || E == EPI_BIAS || E == EPI_BIAS_GELU || E == EPI_BIAS_RESID ||
                            E == EPI_DUMP_I;
-    if (!small_ring4(M, w.N)) return gemm::run<Small3, E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream);
+    if (!small_ring4(M, w.N)) return gemm::run<Small3, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
     if constexpr (plain) {
-        if (small_rows32(M, w.N)) return gemm::run<Small4T, E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream);
-        return gemm::run<Small4W, E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream);
+        if (small_rows32(M, w.N)) return gemm::run<Small4T, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        return gemm::run<Small4W, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
     }
-    return gemm::run<Small4, E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream);
+    return gemm::run<Small4, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
 }
 
 hipError_t launch_gemm_f16(const _Float16 *w16, int64_t K_pad, int64_t N, const _Float16 *x16,

@@ -15,7 +15,7 @@ constexpr int64_t MAX_SEG_LEN = 4096;
 
 // Device view of a repacked Q8_0 weight (K_pad, N).
 struct WeightView {
-    const int8_t *qs;     // N rows of K_pad int8 (16-byte aligned)
+    const int8_t *qs;     // N rows of K_pad int8, ld_qs bytes apart (16-byte aligned)
     // KB rows of ldT fp16 bits of d (transposed); within each group of 64
     // columns, column c + j (j < 32) sits at 2 j and c + 32 + j at 2 j + 1,
     // so one 32-bit word holds the scales of columns j and j + 32
@@ -23,7 +23,16 @@ struct WeightView {
     int64_t ldT;          // >= round_up(N, GEMM_BN)
     int64_t K_pad;        // multiple of 32
     int64_t N;
+    int64_t ld_qs;        // >= K_pad, multiple of 16
 };
+
+// Row stride of int8 quants that the GEMM reads fastest: whole 128-byte cache
+// lines, so that the 128 bytes (4 blocks) of a row that one of its loads
+// takes lie in one line and not two (29 against 17 cycles of the vector
+// memory path per 1 KB, measured at strides 4,320 and 1,152).
+inline int64_t gemm_ld_q(int64_t K_pad) {
+    return K_pad > (1 << 23) ? K_pad : (K_pad + 127) / 128 * 128;  // (a tile's rows stay within 31 bits)
+}
 
 // Column tile of the GEMM; the transposed weight scales are padded to it.
 constexpr int64_t GEMM_BN = 128;
@@ -60,11 +69,11 @@ struct EpiParams {
     _Float16      *q, *k, *vt;
     const int32_t *rowmap;
     int            n_head, d_head, d_pad, dv_pad, len_pad;
-    // EPI_GELU_Q81: quants [M][q_kpad] (columns N..q_kpad-1 quantize zeros)
-    // and ds words [M][q_ldds]
+    // EPI_GELU_Q81: quants [M][q_kpad] (columns N..q_kpad-1 quantize zeros),
+    // rows q_ld bytes apart (0: q_kpad), and ds words [M][q_ldds]
     int8_t   *q_out8;
     uint32_t *q_ds;
-    int64_t   q_kpad, q_ldds;
+    int64_t   q_kpad, q_ldds, q_ld;
     // EPI_GELU_F16: f16 rows [M][h_ld], columns N..h_kpad-1 written as zero
     _Float16 *h_out;
     int64_t   h_ld, h_kpad;
@@ -81,14 +90,15 @@ hipError_t launch_quantize_q8_1(const float *x, int64_t K, int64_t M, int64_t ld
 
 // a2: raw block_q8_0 (N rows of K_pad/32 34-byte blocks, device) -> WeightView
 // planes
-hipError_t launch_repack_q8_0(const void *raw, int64_t K_pad, int64_t N, int8_t *qs,
+hipError_t launch_repack_q8_0(const void *raw, int64_t K_pad, int64_t N, int8_t *qs, int64_t ld_qs,
                               uint16_t *dT, int64_t ldT, hipStream_t stream);
 
 // a3: Y = W x X(Q8_1) with epilogue, on int8 MFMA (s2x_gemm.hip).  xq: int8
-// quants [M][K_pad] (16-byte aligned), xds: ds words [M][ld_ds].
+// quants [M][K_pad], rows ldx bytes apart (0: K_pad; a multiple of 16;
+// 16-byte aligned), xds: ds words [M][ld_ds].
 hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xds, int64_t ld_ds,
                        int64_t M, float *y, int64_t ldy, const EpiParams &epi,
-                       hipStream_t stream);
+                       hipStream_t stream, int64_t ldx = 0);
 
 // F16 weights (the converter's type for matrices whose K is not a multiple
 // of 32, e.g. ffn_down): Y = W16 x f16(X) with f32 accumulation on f16 MFMA.
@@ -104,7 +114,7 @@ hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xd
 hipError_t launch_gemm_split_k(const WeightView &w, const int8_t *xq, const uint32_t *xds,
                                int64_t ld_ds, int64_t M, float *y, int64_t ldy,
                                const EpiParams &epi, int n_split, float *part,
-                               hipStream_t stream);
+                               hipStream_t stream, int64_t ldx = 0);
 
 hipError_t launch_gemm_f16(const _Float16 *w16, int64_t K_pad, int64_t N, const _Float16 *x16,
                            int64_t M, float *y, int64_t ldy, const EpiParams &epi,

@@ -86,7 +86,7 @@ __device__ __forceinline__ int64_t dw_pos(int64_t n) {
 
 __global__ __launch_bounds__(256) void k_repack_q8_0(const uint8_t *__restrict__ raw,
                                                      int64_t n_blocks, int64_t KB,
-                                                     int8_t *__restrict__ qs,
+                                                     int8_t *__restrict__ qs, int64_t ld_qs,
                                                      uint16_t *__restrict__ dT, int64_t ldT) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_blocks) return;
@@ -96,7 +96,7 @@ __global__ __launch_bounds__(256) void k_repack_q8_0(const uint8_t *__restrict__
     uint32_t w[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) w[j] = (uint32_t)src[1 + 2 * j] | ((uint32_t)src[2 + 2 * j] << 16);
-    uint4 *dst = reinterpret_cast<uint4 *>(qs + i * QK);
+    uint4 *dst = reinterpret_cast<uint4 *>(qs + n * ld_qs + kb * QK);
     dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
     dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
 }
@@ -110,12 +110,12 @@ __global__ __launch_bounds__(256) void k_zero_pad_cols(uint16_t *__restrict__ dT
     dT[(i / w) * ldT + dw_pos(N + i % w)] = 0;
 }
 
-hipError_t launch_repack_q8_0(const void *raw, int64_t K_pad, int64_t N, int8_t *qs,
+hipError_t launch_repack_q8_0(const void *raw, int64_t K_pad, int64_t N, int8_t *qs, int64_t ld_qs,
                               uint16_t *dT, int64_t ldT, hipStream_t stream) {
     const int64_t KB = K_pad / QK, nb = N * KB;
     if (nb == 0) return hipSuccess;
     hipLaunchKernelGGL(k_repack_q8_0, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0,
-                       stream, reinterpret_cast<const uint8_t *>(raw), nb, KB, qs, dT, ldT);
+                       stream, reinterpret_cast<const uint8_t *>(raw), nb, KB, qs, ld_qs, dT, ldT);
     if (ldT > N)
         hipLaunchKernelGGL(k_zero_pad_cols, dim3((unsigned)((KB * (ldT - N) + 255) / 256)),
                            dim3(256), 0, stream, dT, KB, N, ldT);
