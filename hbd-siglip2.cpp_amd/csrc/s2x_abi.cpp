@@ -304,13 +304,19 @@ int s2x_mul_mat_f16_f32(const void *w_raw, int64_t K, int64_t N, const float *x,
     const int64_t K_pad = round_up_i(K, QK_);
     uint8_t *ws = (uint8_t *)workspace;
     hipStream_t s = (hipStream_t)stream;
-    _Float16 *w16 = (_Float16 *)(ws + L.w_off), *x16 = (_Float16 *)(ws + L.xq_off);
-    hipError_t e = launch_repack_f16(w_raw, K, N, K_pad, w16, s);
-    if (e != hipSuccess) return hip_fail(e, "repack launch");
-    e = launch_f32_to_f16(x, K, M, ldx, K_pad, x16, s);
+    // The GEMM reads the raw weight rows in place where they are 16-byte
+    // aligned; X then has the whole workspace for rows of whole 128-byte
+    // lines, if those fit.
+    const bool w_direct = K % 8 == 0 && aligned(w_raw, 16);
+    const int64_t ld_line = round_up_i(K, 64);
+    const bool x_lines = w_direct && (size_t)(M * ld_line * 2) <= L.total;
+    const int64_t ldx16 = x_lines ? ld_line : K_pad, ldw = w_direct ? K : K_pad;
+    _Float16 *x16 = (_Float16 *)(ws + (x_lines ? 0 : L.xq_off));
+    _Float16 *w16 = w_direct ? (_Float16 *)const_cast<void *>(w_raw) : (_Float16 *)(ws + L.w_off);
+    hipError_t e = launch_f16_operands(x, K, M, ldx, x16, ldx16, w_direct ? nullptr : w_raw, N, w16, ldw, s);
     if (e != hipSuccess) return hip_fail(e, "convert launch");
     EpiParams p{EPI_NONE, nullptr, nullptr, 0, 0, 0};
-    e = launch_gemm_f16(w16, K_pad, N, x16, M, y, N, p, s);
+    e = launch_gemm_f16(w16, ldw, K, N, x16, ldx16, M, y, N, p, s);
     return e == hipSuccess ? S2X_OK : hip_fail(e, "gemm launch");
 }
 

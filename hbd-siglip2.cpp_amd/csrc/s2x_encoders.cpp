@@ -123,17 +123,20 @@ int upload_q8(const void *raw, int64_t K_pad, int64_t N, hipStream_t s, s2x_weig
     return weight_upload(raw, true, K_pad, N, s, w);
 }
 
-// F16 matrix (N rows of K halves, host) -> device rows of K_pad halves, zero
-// past K
+// Row stride (halves) of f16 operands of the towers: whole 128-byte lines
+int64_t f16_ld(int64_t K_pad) { return (K_pad + 63) / 64 * 64; }
+
+// F16 matrix (N rows of K halves, host) -> device rows of f16_ld(K_pad)
+// halves, zero past K
 int upload_f16(const void *raw, int64_t K, int64_t K_pad, int64_t N, _Float16 **dev,
                const char *what) {
     *dev = nullptr;
     if (!raw) return fail(S2X_ERR_INVALID_ARG, "missing tensor %s", what);
-    const size_t bytes = sizeof(_Float16) * (size_t)(N * K_pad);
+    const size_t ld = (size_t)f16_ld(K_pad), bytes = sizeof(_Float16) * (size_t)N * ld;
     if (hipMalloc(reinterpret_cast<void **>(dev), bytes) != hipSuccess)
         return fail(S2X_ERR_OOM, "hipMalloc for %s failed", what);
     S2X_HIP_TRY(hipMemset(*dev, 0, bytes));
-    S2X_HIP_TRY(hipMemcpy2D(*dev, (size_t)K_pad * 2, raw, (size_t)K * 2, (size_t)K * 2, (size_t)N,
+    S2X_HIP_TRY(hipMemcpy2D(*dev, ld * 2, raw, (size_t)K * 2, (size_t)K * 2, (size_t)N,
                             hipMemcpyHostToDevice));
     return S2X_OK;
 }
@@ -141,7 +144,7 @@ int upload_f16(const void *raw, int64_t K, int64_t K_pad, int64_t N, _Float16 **
 // ffn_down: a Q8_0 weight, or F16 rows (the converter's type for K % 32 != 0)
 struct DownW {
     s2x_weight *q8 = nullptr;
-    _Float16 *f16 = nullptr;  // N rows of K_pad halves
+    _Float16 *f16 = nullptr;  // N rows of f16_ld(K_pad) halves
     void release() {
         s2x_weight_destroy(q8);
         if (f16) (void)hipFree(f16);
@@ -376,11 +379,11 @@ struct Tower {
         if (down.f16) {
             EpiParams ep{EPI_GELU_F16, up_b, nullptr, 0, 0, 0};
             ep.h_out = h16.as<_Float16>();
-            ep.h_ld = ep.h_kpad = F_pad;
+            ep.h_kpad = F_pad;
+            ep.h_ld = f16_ld(F_pad);
             S2X_TRY(gemm(up, M, nullptr, 0, ep, H));
-            const hipError_t e = launch_gemm_f16(down.f16, F_pad, H, h16.as<_Float16>(), M, y, H,
-                                                 EpiParams{EPI_BIAS_RESID, down_b, resid, H, 0, 0},
-                                                 stream);
+            const hipError_t e = launch_gemm_f16(down.f16, f16_ld(F_pad), F_pad, H, h16.as<_Float16>(), ep.h_ld, M,
+                                                 y, H, EpiParams{EPI_BIAS_RESID, down_b, resid, H, 0, 0}, stream);
             return e == hipSuccess ? S2X_OK : hip_fail(e, "f16 gemm launch");
         }
         EpiParams ep{EPI_GELU_Q81, up_b, nullptr, 0, 0, 0};
@@ -421,7 +424,7 @@ struct Tower {
         S2X_TRY(ensure(qs, (size_t)(M * kmax), stream));
         S2X_TRY(ensure(ds, sizeof(uint32_t) * (size_t)(M * (kmax / QK_)), stream));
         if (down_f16) {
-            S2X_TRY(ensure(h16, sizeof(_Float16) * (size_t)(M * F_pad), stream));
+            S2X_TRY(ensure(h16, sizeof(_Float16) * (size_t)(M * f16_ld(F_pad)), stream));
         } else {
             S2X_TRY(ensure(qs2, (size_t)(M * gemm_ld_q(F_pad)), stream));
             S2X_TRY(ensure(ds2, sizeof(uint32_t) * (size_t)(M * (F_pad / QK_)), stream));

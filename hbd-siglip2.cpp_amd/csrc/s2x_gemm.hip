@@ -261,21 +261,36 @@ __device__ __forceinline__ void epilogue(float (&acc)[TM][TN][16], float scale, 
             }
     } else if constexpr (EPI == EPI_GELU_F16) {
         // GELU(mm + bias) rounded to f16, rows of h_kpad halves (columns
-        // N .. h_kpad - 1 zero): the f16 activation of an F16 weight
+        // N .. h_kpad - 1 zero): the f16 activation of an F16 weight.  Each
+        // 32 x 64 half goes through LDS so that 8 columns of a row leave as
+        // one 16-byte store where the rows are 16-byte aligned.
+        constexpr int P = 72;  // halves per scratch row
+        _Float16 *scr = reinterpret_cast<_Float16 *>(wscr);
+        const bool vec = epi.h_ld % 8 == 0 && (reinterpret_cast<uintptr_t>(epi.h_out) & 15) == 0;  // uniform
 #pragma unroll
-        for (int a = 0; a < TM; ++a)
+        for (int a = 0; a < TM; ++a) {
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const int n = nw + b * 32 + lr;
-                if (n >= epi.h_kpad) continue;
+            for (int b = 0; b < 2; ++b)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = mw + a * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
-                    if (m < M)
-                        epi.h_out[(int64_t)m * epi.h_ld + n] =
-                            n < N ? f32_to_f16(gelu_tanh(fmaf(acc[a][b][r], scale, bias_v[b]))) : (_Float16)0.0f;
+                for (int r = 0; r < 16; ++r)
+                    scr[(8 * (r >> 2) + 4 * lh + (r & 3)) * P + b * 32 + lr] =
+                        nw + b * 32 + lr < N ? f32_to_f16(gelu_tanh(fmaf(acc[a][b][r], scale, bias_v[b])))
+                                             : (_Float16)0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int id = lane + 64 * i, row = id >> 3, c = (id & 7) * 8;
+                const int m = mw + a * 32 + row, n = nw + c;
+                if (m >= M || n >= epi.h_kpad) continue;  // (h_kpad is a multiple of 32: whole chunks)
+                _Float16 *dst = epi.h_out + (int64_t)m * epi.h_ld + n;
+                const v8h v = *reinterpret_cast<const v8h *>(scr + row * P + c);
+                if (vec) {
+                    *reinterpret_cast<v8h *>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) dst[j] = v[j];
                 }
             }
+        }
     } else if constexpr (EPI == EPI_QKV) {
         // (mm + bias) in f32, then f16, into Q / K [seg][head][pos][d_pad]
         // or V^T [seg][head][dv_pad][pos]; padding slots are not written
@@ -939,7 +954,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // Epilogue.  The LDS is free scratch once the last (empty) stage's DMA
     // has landed and every wave has read its last fragments.
     // ----------------------------------------------------------------------
-    if constexpr (EPI == EPI_GELU_Q81 || EPI == EPI_QKV) {
+    if constexpr (EPI == EPI_GELU_Q81 || EPI == EPI_GELU_F16 || EPI == EPI_QKV) {
         wait_vm<0>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
@@ -978,149 +993,189 @@ hipError_t run(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_
 // ---------------------------------------------------------------------------
 // F16 weight x f16 activation, f32 accumulation (GGML_OP_MUL_MAT with an
 // F16 weight, as the reference's converter stores ffn_down: K = 4304 is
-// not a multiple of 32).  Same tiles, waves, tile order and LDS-DMA ring as
-// k_gemm; a K block is 32 halves (64-byte rows, four 16-byte chunks, chunk
-// c of row r at position c ^ ((r >> 2) & 3)), two v_mfma_f32_32x32x16_f16
-// per subtile accumulate straight into the outputs: no scales, no VALU.
+// not a multiple of 32).  A stage is 64 halves (a 128-byte line) of BM
+// rows of X and BN of W, brought by LDS DMA into a ring of NS stages, two of
+// them in flight while one is used; a fragment pair is read one step ahead
+// of its MFMAs, also over the stage's barrier.  A CU's LDS-DMA path (about
+// 64 bytes a cycle) and its matrix pipes bound it alike: 128 x 128 tiles
+// need 32 KB per 512 matrix cycles.  Its instructions therefore go between
+// the MFMAs, two per step: issued in one burst after the barrier they hold
+// the wave, and its matrix pipe, for about as long as the MFMAs take (M =
+// 2,916, K = 4,304, N = 1,152: 40.0 us, spread 37.9).  Before, with a ring of
+// two half-line stages and no fragment ahead, that product with its operand
+// conversions took 83.6 us, now 53.9; X in rows of whole lines and the raw W
+// read in place where it is aligned are part of it (W in whole lines, as the
+// towers hold it: 33.9 us).
 // ---------------------------------------------------------------------------
+// BM x BN tiles of WM x WN waves, each 32 TM x 32 TN outputs; stages of 64
+// halves (128 bytes a row) in a ring of NS.
+template <int TM_, int TN_, int WM_, int WN_, int NS_>
 struct CfgH {
-    static constexpr int BM = 128, KS = 2, NS = 2, NWAVE = 8, NT = NWAVE * WAVE;
-    static constexpr int XQ = 0, WQ = XQ + KS * BM * 64, STAGE = WQ + KS * BN * 64;
-    static constexpr int LDS_BYTES = NS * STAGE;  // 64 KiB: two workgroups per CU
-    static constexpr int DMA_N = 2 * (KS * BM / 16) / NWAVE;  // 16 rows of a block per instruction
-    static_assert(NWAVE * EPI_SCRATCH <= LDS_BYTES, "epilogue scratch");
+    static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, NS = NS_;
+    static constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, NWAVE = WM * WN, NT = NWAVE * WAVE;
+    static constexpr int XQ = 0, WQ = BM * 128, STAGE = WQ + BN * 128, LDS_BYTES = NS * STAGE;
+    static constexpr int QPX = BM / 8 / NWAVE, QPW = BN / 8 / NWAVE, DPS = QPX + QPW;  // DMA per wave and stage
+    static constexpr int WG_PER_CU = 163840 / LDS_BYTES >= 2 ? 2 : 1;
+    static constexpr int WPE = (WG_PER_CU * NWAVE + 3) / 4;  // waves per SIMD
+    static_assert(QPX * NWAVE * 8 == BM && QPW * NWAVE * 8 == BN, "DMA split");
+    static_assert(NS >= 3 && LDS_BYTES <= 163840, "ring");
 };
 
-__device__ __forceinline__ int swz4(int r) { return (r >> 2) & 3; }
-
-template <int EPI>
-__global__ __launch_bounds__(CfgH::NT) __attribute__((amdgpu_waves_per_eu(4))) void k_gemm_f16(
-    const uint8_t *__restrict__ xh, const uint8_t *__restrict__ wh, int M, int N, int KB,
-    float *__restrict__ y, int64_t ldy, EpiParams epi) {
-    using C = CfgH;
-    constexpr int BM = C::BM, KS = C::KS, STAGE = C::STAGE, XQ = C::XQ, WQ = C::WQ;
+template <class C, int EPI>
+__global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE))) void k_gemm_f16(
+    const uint8_t *__restrict__ xh, int64_t ldx, const uint8_t *__restrict__ wh, int64_t ldw, int M, int N,
+    int KC, float *__restrict__ y, int64_t ldy, EpiParams epi) {
+    constexpr int BM = C::BM, BN_ = C::BN, TM = C::TM, TN = C::TN, NS = C::NS, STAGE = C::STAGE;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / C::WN, wn = wave % C::WN;
     const int lr = lane & 31, lh = lane >> 5;
-    const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
+    const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN_ - 1) / BN_;
     int tm, tn;
     tile_of(xcd_linear(blockIdx.x, gridDim.x), m_tiles, n_tiles, tm, tn);
-    const int m0 = tm * BM, n0 = tn * BN;
-    const int n_st = (KB + KS - 1) / KS;
-    const int64_t row_bytes = (int64_t)KB * 64;
+    const int m0 = tm * BM, n0 = tn * BN_;
+    const int n_st = (KC + 7) / 8;
 
-    // DMA: a stage is KS blocks x 128 rows of X and of W, 16 rows of one
-    // block per instruction (lane: row lane / 4, chunk position lane % 4);
-    // waves 0-3 fetch X, 4-7 W, instruction t of wave w: block t % KS, rows
-    // 16 (G (w % 4) + t / KS) .. + 15, G = DMA_N / KS row groups per wave
-    const int kind = wave >> 2;
-    const __amdgpu_buffer_rsrc_t src_live = kind == 0
-        ? __builtin_amdgcn_make_buffer_rsrc((void *)(xh + (int64_t)m0 * row_bytes), (short)0,
-                                            clip32((int64_t)(M - m0) * row_bytes), BUF_DW3)
-        : __builtin_amdgcn_make_buffer_rsrc((void *)(wh + (int64_t)n0 * row_bytes), (short)0,
-                                            clip32((int64_t)(N - n0) * row_bytes), BUF_DW3);
+    // One DMA instruction brings a stage's 128 bytes of 8 rows; the eight
+    // 16-byte chunks of row r lie at positions c ^ swz8(r), as in k_gemm.
+    // Chunks past KC (the last stage) and rows past M or N are out of the
+    // buffer's range through the per-lane offset: they arrive as zeros and
+    // nothing past a row's KC chunks is read.
+    const __amdgpu_buffer_rsrc_t xr_live = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(xh + (int64_t)m0 * ldx), (short)0, clip32((int64_t)(M - m0 - 1) * ldx + KC * 16), BUF_DW3);
+    const __amdgpu_buffer_rsrc_t wr_live = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(wh + (int64_t)n0 * ldw), (short)0, clip32((int64_t)(N - n0 - 1) * ldw + KC * 16), BUF_DW3);
     const __amdgpu_buffer_rsrc_t none = __builtin_amdgcn_make_buffer_rsrc((void *)xh, (short)0, 0, BUF_DW3);
-    uint32_t voff[C::DMA_N];
+    const int c0 = (lane & 7) ^ (lane >> 3);  // the lane's chunk in instructions of even row groups; c0 ^ 1 in odd ones
+    uint32_t vx[C::QPX], vw[C::QPW];
 #pragma unroll
-    for (int t = 0; t < C::DMA_N; ++t) {
-        const int r = 16 * (C::DMA_N / KS * (wave & 3) + t / KS) + (lane >> 2);
-        voff[t] = (uint32_t)(r * row_bytes) + (uint32_t)(((lane & 3) ^ swz4(r)) * 16);
+    for (int t = 0; t < C::QPX; ++t) {
+        const int i = C::QPX * wave + t;
+        vx[t] = (uint32_t)((8 * i + (lane >> 3)) * ldx) + (uint32_t)((c0 ^ (i & 1)) * 16);
     }
-    // blocks past KB (an odd KB's last stage, every block of a stage past
-    // the last) through the zero-size buffer: nothing past the planes is
-    // addressed
-    auto issue = [&](int g) {
-        uint8_t *sb = lds + (g & 1) * STAGE + (kind == 0 ? XQ : WQ);
-        const uint32_t k0 = (uint32_t)(g * KS);
 #pragma unroll
-        for (int t = 0; t < C::DMA_N; ++t) {
-            const int j = t % KS, grp = C::DMA_N / KS * (wave & 3) + t / KS;
-            dma16((int)k0 + j < KB ? src_live : none, voff[t], (k0 + j) * 64,
-                  sb + j * BM * 64 + grp * 1024);
-        }
-    };
-    auto arrive = [&](int g) {
-        wait_vm<0>();
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        issue(g + 1);
-    };
-
-    const int xrow = wm * 32 + lr;
-    int a_off[2], b_off[2][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        a_off[h] = XQ + xrow * 64 + (((2 * h + lh) ^ swz4(xrow)) * 16);
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const int wc = wn * 64 + b * 32 + lr;
-            b_off[b][h] = WQ + wc * 64 + (((2 * h + lh) ^ swz4(wc)) * 16);
-        }
+    for (int t = 0; t < C::QPW; ++t) {
+        const int i = C::QPW * wave + t;
+        vw[t] = (uint32_t)((8 * i + (lane >> 3)) * ldw) + (uint32_t)((c0 ^ (i & 1)) * 16);
     }
-    v16f acc_v[2] = {};
-    auto block = [&](const uint8_t *sb, int j) {
-        v8h a[2], bq[2][2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            a[h] = *reinterpret_cast<const v8h *>(sb + a_off[h] + j * BM * 64);
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-                bq[b][h] = *reinterpret_cast<const v8h *>(sb + b_off[b][h] + j * BN * 64);
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-                acc_v[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[h], bq[b][h], acc_v[b], 0, 0, 0);
+    // instructions [lo, hi) of stage g's DPS into ring slot `slot`; a stage
+    // past the last goes through a zero-size buffer
+    auto issue = [&](int g, int slot, auto lo_c, auto hi_c) {
+        constexpr int LO = decltype(lo_c)::value, HI = decltype(hi_c)::value;
+        uint8_t *sb = lds + slot * STAGE;
+        const bool live = g < n_st;
+        const __amdgpu_buffer_rsrc_t xr = live ? xr_live : none, wr = live ? wr_live : none;
+        const int left = KC - 8 * g;  // chunks of this stage
+        const uint32_t k0 = live ? (uint32_t)g * 128u : 0u;
+        static_for<HI - LO>([&](auto tc) {
+            constexpr int t = LO + decltype(tc)::value;
+            if constexpr (t < C::QPX) {
+                const int i = C::QPX * wave + t;
+                dma16(xr, (c0 ^ (i & 1)) < left ? vx[t] : OOB_OFF, k0, sb + C::XQ + i * 1024);
+            } else {
+                const int i = C::QPW * wave + t - C::QPX;
+                dma16(wr, (c0 ^ (i & 1)) < left ? vw[t - C::QPX] : OOB_OFF, k0, sb + C::WQ + i * 1024);
+            }
+        });
     };
+    using std::integral_constant;
+    const integral_constant<int, 0> i_0{};
+    const integral_constant<int, C::DPS> i_n{};
 
-    issue(0);
-    arrive(0);
+    struct FragH {
+        v8h a[TM], b[TN];
+    };
+    const int a_off = C::XQ + (wm * 32 * TM + lr) * 128 + ((lh ^ swz8(lr)) * 16);
+    const int b_off = C::WQ + (wn * 32 * TN + lr) * 128 + ((lh ^ swz8(lr)) * 16);
+    auto load_frag = [&](const uint8_t *sb, int s, FragH &f) {
+#pragma unroll
+        for (int a = 0; a < TM; ++a) f.a[a] = *reinterpret_cast<const v8h *>(sb + (a_off ^ (s * 32)) + a * 4096);
+#pragma unroll
+        for (int b = 0; b < TN; ++b) f.b[b] = *reinterpret_cast<const v8h *>(sb + (b_off ^ (s * 32)) + b * 4096);
+    };
+    v16f acc_v[TM][TN] = {};
+    // one step of 16 halves: its MFMAs with DMA instructions [LO, HI) of
+    // stage g spread between them (issued in one burst they hold the wave,
+    // and with it the matrix pipe, until the memory path has taken them)
+    auto step = [&](const FragH &f, int g, int slot, auto lo_c, auto hi_c) {
+        constexpr int LO = decltype(lo_c)::value, HI = decltype(hi_c)::value, NM = TM * TN;
+        static_for<NM>([&](auto kc) {
+            constexpr int k = decltype(kc)::value, a = k / TN, b = k % TN;
+            constexpr int l = LO + (HI - LO) * k / NM, h = LO + (HI - LO) * (k + 1) / NM;
+            if constexpr (h > l) issue(g, slot, integral_constant<int, l>{}, integral_constant<int, h>{});
+            acc_v[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[a], f.b[b], acc_v[a][b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    // step s of a stage issues instructions [part(s), part(s + 1))
+    constexpr auto part = [](int s) { return C::DPS * s / 4; };
+
+    static_for<NS - 1>([&](auto sc) { issue(decltype(sc)::value, decltype(sc)::value, i_0, i_n); });
+    wait_vm<(NS - 2) * C::DPS>();
+    asm volatile("s_barrier" ::: "memory");
+    FragH F[2];
+    load_frag(lds, 0, F[0]);
+    int slot = 0;  // stage g's; stage g + NS - 1 goes into the one before
     for (int g = 0; g < n_st - 1; ++g) {
-        const uint8_t *sb = lds + (g & 1) * STAGE;
-#pragma unroll
-        for (int j = 0; j < KS; ++j) block(sb, j);
-        arrive(g + 1);
+        const uint8_t *sb = lds + slot * STAGE;
+        const int nslot = slot + 1 == NS ? 0 : slot + 1, pslot = slot == 0 ? NS - 1 : slot - 1;
+        static_for<3>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            load_frag(sb, s + 1, F[(s + 1) & 1]);
+            step(F[s & 1], g + NS - 1, pslot, integral_constant<int, part(s)>{}, integral_constant<int, part(s + 1)>{});
+        });
+        // every wave has its last fragments of stage g (its slot is free from
+        // here on), stage g + 1 has landed
+        wait_vm<(NS - 3) * C::DPS + part(3)>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        load_frag(lds + nslot * STAGE, 0, F[0]);
+        step(F[1], g + NS - 1, pslot, integral_constant<int, part(3)>{}, i_n);
+        slot = nslot;
     }
     {
-        const uint8_t *sb = lds + ((n_st - 1) & 1) * STAGE;
-        const int nb = KB - (n_st - 1) * KS;
-#pragma unroll
-        for (int j = 0; j < KS; ++j)
-            if (j < nb) block(sb, j);
+        const uint8_t *sb = lds + slot * STAGE;
+        const int nk = (KC - 8 * (n_st - 1) + 1) / 2;  // 1 .. 4 steps of 16 halves
+        step(F[0], 0, 0, i_0, i_0);
+        static_for<3>([&](auto sc) {
+            constexpr int s = decltype(sc)::value + 1;
+            if (s < nk) {
+                load_frag(sb, s, F[0]);
+                step(F[0], 0, 0, i_0, i_0);
+            }
+        });
     }
 
-    float acc[1][2][16];
-    float bias_v[2];
+    float acc[TM][TN][16];
+    float bias_v[TN];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const int n = n0 + wn * 64 + b * 32 + lr;
+    for (int b = 0; b < TN; ++b) {
+        const int n = n0 + wn * 32 * TN + b * 32 + lr;
         bias_v[b] = EPI != EPI_NONE && n < N ? epi.bias[n] : 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[0][b][r] = acc_v[b][r];
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = acc_v[a][b][r];
     }
-    epilogue<1, 2, EPI>(acc, 1.0f, bias_v, lane, m0 + wm * 32, n0 + wn * 64, M, N, y, ldy, epi,
-                     lds + wave * EPI_SCRATCH);
+    epilogue<TM, TN, EPI>(acc, 1.0f, bias_v, lane, m0 + wm * 32 * TM, n0 + wn * 32 * TN, M, N, y, ldy, epi, nullptr);
     wait_vm<0>();
 }
 
-template <int EPI>
-hipError_t run_f16(const _Float16 *w16, int64_t K_pad, int64_t N, const _Float16 *x16, int64_t M,
+template <class C, int EPI>
+hipError_t run_f16(const _Float16 *w16, int64_t ldw, int64_t K, int64_t N, const _Float16 *x16, int64_t ldx, int64_t M,
                    float *y, int64_t ldy, const EpiParams &epi, hipStream_t stream) {
-    auto kern = k_gemm_f16<EPI>;
+    auto kern = k_gemm_f16<C, EPI>;
     static bool attr_set = false;
     if (!attr_set) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                 CfgH::LDS_BYTES);
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES);
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    const int64_t tiles = ((M + CfgH::BM - 1) / CfgH::BM) * ((N + BN - 1) / BN);
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(CfgH::NT), CfgH::LDS_BYTES, stream,
-                       reinterpret_cast<const uint8_t *>(x16), reinterpret_cast<const uint8_t *>(w16),
-                       (int)M, (int)N, (int)(K_pad / QK), y, ldy, epi);
+    const int64_t tiles = ((M + C::BM - 1) / C::BM) * ((N + C::BN - 1) / C::BN);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(C::NT), C::LDS_BYTES, stream,
+                       reinterpret_cast<const uint8_t *>(x16), ldx * 2, reinterpret_cast<const uint8_t *>(w16),
+                       ldw * 2, (int)M, (int)N, (int)((K + 7) / 8), y, ldy, epi);
     return hipGetLastError();
 }
 
@@ -1499,22 +1554,49 @@ static hipError_t run_small(const WeightView &w, const int8_t *xq, int64_t ldx, 
     return gemm::run<Small4, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
 }
 
-hipError_t launch_gemm_f16(const _Float16 *w16, int64_t K_pad, int64_t N, const _Float16 *x16,
-                           int64_t M, float *y, int64_t ldy, const EpiParams &epi,
+// The form of an F16 product, by tiles per round of the 256 CUs (every form
+// gives the same bits).  Small: 64 x 64 tiles, two workgroups a CU, while all
+// of them are resident at once (M = 729, K = 4320, N = 1152: 18 us against
+// 33 in 128 x 128 tiles; at 648 tiles, M = 729, K = 1152, N = 3456: 14.6
+// against 12.4).  Above that 128 x 128 tiles, or 256 x 128 where that takes
+// fewer rounds by more than the 1.6 x that a round of them is longer: M =
+// 3645, K = 4320, N = 1152 (2 rounds or 1) 63 against 51 us, M = 8640 (3 or
+// 2) 103 against 107, M = 23,328 (7 or 4) 301 against 257.
+using SmallH = gemm::CfgH<1, 1, 2, 2, 4>;
+using MidH = gemm::CfgH<1, 2, 4, 2, 4>;
+using WideH = gemm::CfgH<2, 2, 4, 2, 3>;
+
+template <int E>
+static hipError_t run_f16_form(const _Float16 *w16, int64_t ldw, int64_t K, int64_t N, const _Float16 *x16,
+                               int64_t ldx, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
+                               hipStream_t stream) {
+    const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const auto rounds = [&](int64_t t) { return (t + 255) / 256; };
+    if (tiles(SmallH::BM, SmallH::BN) <= 512)
+        return gemm::run_f16<SmallH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
+    if (8 * rounds(tiles(WideH::BM, WideH::BN)) < 5 * rounds(tiles(MidH::BM, MidH::BN)) &&
+        WideH::BM * ldx * 2 <= 0x7fffffff)
+        return gemm::run_f16<WideH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
+    return gemm::run_f16<MidH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
+}
+
+hipError_t launch_gemm_f16(const _Float16 *w16, int64_t ldw, int64_t K, int64_t N, const _Float16 *x16,
+                           int64_t ldx, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
                            hipStream_t stream) {
     if (M == 0 || N == 0) return hipSuccess;
-    if (!w16 || !x16 || !y || K_pad <= 0 || K_pad % QK || M > (1 << 30) || N > (1 << 30) ||
-        ((uintptr_t)w16 & 15) || ((uintptr_t)x16 & 15) || (int64_t)gemm::CfgH::BM * K_pad * 2 > 0x7fffffff ||
-        gemm::CfgH::BM * ldy * 4 > 0x7fffffff)
+    const int64_t K8 = (K + 7) / 8 * 8;
+    if (!w16 || !x16 || !y || K <= 0 || ldw < K8 || ldx < K8 || ldw % 8 || ldx % 8 || M > (1 << 30) ||
+        N > (1 << 30) || ((uintptr_t)w16 & 15) || ((uintptr_t)x16 & 15) || 128 * ldw * 2 > 0x7fffffff ||
+        128 * ldx * 2 > 0x7fffffff || 128 * ldy * 4 > 0x7fffffff)
         return hipErrorInvalidValue;
     switch (epi.kind) {
-    case EPI_NONE: return gemm::run_f16<EPI_NONE>(w16, K_pad, N, x16, M, y, ldy, epi, stream);
-    case EPI_BIAS: return gemm::run_f16<EPI_BIAS>(w16, K_pad, N, x16, M, y, ldy, epi, stream);
+    case EPI_NONE: return run_f16_form<EPI_NONE>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
+    case EPI_BIAS: return run_f16_form<EPI_BIAS>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
     case EPI_BIAS_RESID:
         if (!epi.resid || epi.ld_resid < N || epi.resid_rows < 0 ||
-            (epi.resid_rows > 0 ? epi.resid_rows : gemm::CfgH::BM) * epi.ld_resid * 4 > 0x7fffffff)
+            (epi.resid_rows > 0 ? epi.resid_rows : 128) * epi.ld_resid * 4 > 0x7fffffff)
             return hipErrorInvalidValue;
-        return gemm::run_f16<EPI_BIAS_RESID>(w16, K_pad, N, x16, M, y, ldy, epi, stream);
+        return run_f16_form<EPI_BIAS_RESID>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
     default: return hipErrorInvalidValue;
     }
 }

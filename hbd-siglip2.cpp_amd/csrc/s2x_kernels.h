@@ -100,10 +100,6 @@ hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xd
                        int64_t M, float *y, int64_t ldy, const EpiParams &epi,
                        hipStream_t stream, int64_t ldx = 0);
 
-// F16 weights (the converter's type for matrices whose K is not a multiple
-// of 32, e.g. ffn_down): Y = W16 x f16(X) with f32 accumulation on f16 MFMA.
-// w16: N rows of K_pad halves, x16: M rows of K_pad halves (both zero past
-// K, 16-byte aligned rows); epilogues NONE, BIAS, BIAS_RESID.
 // The same product as launch_gemm with EPI_NONE / EPI_BIAS_RESID, its K
 // blocks in n_split contiguous ranges of whole 4-block stages (a function of
 // K alone): each range's sum, in block order from zero, goes to a partial
@@ -116,15 +112,19 @@ hipError_t launch_gemm_split_k(const WeightView &w, const int8_t *xq, const uint
                                const EpiParams &epi, int n_split, float *part,
                                hipStream_t stream, int64_t ldx = 0);
 
-hipError_t launch_gemm_f16(const _Float16 *w16, int64_t K_pad, int64_t N, const _Float16 *x16,
-                           int64_t M, float *y, int64_t ldy, const EpiParams &epi,
+// F16 weights (the converter's type for matrices whose K is not a multiple
+// of 32): Y = W16 x f16(X) with f32 accumulation on f16 MFMA.
+// w16: N rows ldw halves apart, x16: M rows ldx halves apart (both multiples
+// of 8, 16-byte aligned), K halves of each used, in steps of 8: a row's
+// halves K .. round_up(K, 8) - 1 are zeros; epilogues NONE, BIAS, BIAS_RESID.
+hipError_t launch_gemm_f16(const _Float16 *w16, int64_t ldw, int64_t K, int64_t N, const _Float16 *x16,
+                           int64_t ldx, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
                            hipStream_t stream);
-// f32 rows (K valid of ldx) -> f16 rows of K_pad halves, zeros past K
-hipError_t launch_f32_to_f16(const float *x, int64_t K, int64_t M, int64_t ldx, int64_t K_pad,
-                             _Float16 *y, hipStream_t stream);
-// raw F16 weight rows (N rows of K halves, device) -> N rows of K_pad halves
-hipError_t launch_repack_f16(const void *raw, int64_t K, int64_t N, int64_t K_pad, _Float16 *w16,
-                             hipStream_t stream);
+// f32 rows (K valid of ldx) -> f16 rows of ldx16 halves and, with raw, raw
+// F16 weight rows (N rows of K halves, device) -> rows of ldw halves; zeros
+// past K
+hipError_t launch_f16_operands(const float *x, int64_t K, int64_t M, int64_t ldx, _Float16 *x16, int64_t ldx16,
+                               const void *raw, int64_t N, _Float16 *w16, int64_t ldw, hipStream_t stream);
 
 // a4: LayerNorm (+ Q8_1).  q may be null (no quantized output), y may be
 // null (no f32 output); at least one is set.

@@ -396,6 +396,35 @@ def test_mul_mat_f16_matches_oracle(orc, M):
                                        ctypes.c_size_t(wsb - 1), stream()) == 4
 
 
+# (M, K, N, elements the weight starts past 16-byte alignment): the three tile
+# forms with ragged rows and columns, K tails inside a 16-half step and inside
+# a 64-half stage, and weights that are repacked (K % 8 or the alignment)
+F16_FORMS = [
+    (1, 8, 1, 0), (65, 24, 70, 0), (130, 72, 129, 0), (64, 4304, 1152, 0),  # 64 x 64 tiles
+    (33, 1001, 40, 0), (70, 136, 65, 1),                                     # repacked weight
+    (16449, 200, 100, 0),                                                    # 128 x 128
+    (32897, 264, 100, 0), (32897, 77, 100, 0),                               # 256 x 128
+]
+
+
+@pytest.mark.parametrize("M,K,N,off", F16_FORMS)
+def test_mul_mat_f16_forms(M, K, N, off):
+    rng = np.random.default_rng(54)
+    w16 = (rng.standard_normal((N, K)) * 0.02).astype(np.float16)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    say(f"F16 mul_mat form M={M} K={K} N={N} off={off}")
+    wd = dev(np.concatenate([np.zeros(off, np.uint16), w16.view(np.uint16).ravel()]))
+    xd = dev(x)
+    wsb = s2x.lib.s2x_mul_mat_f16_workspace_size(K, N, M)
+    ws = torch.full((wsb,), 0xFF, dtype=torch.uint8, device="cuda:0")  # f16 NaNs
+    y = empty((M, N), torch.float32)
+    s2x.call("s2x_mul_mat_f16_f32", ctypes.c_void_p(wd.data_ptr() + 2 * off), K, N, ptr(xd), K, M, ptr(y),
+             ptr(ws), ctypes.c_size_t(wsb), stream())
+    ref = x.astype(np.float16).astype(np.float64) @ w16.astype(np.float64).T
+    # K f32 additions of exact products, in any order
+    assert (np.abs(host(y) - ref) <= K * 2.0 ** -24 * _f16_terms_abs(w16, x)).all()
+
+
 @pytest.mark.parametrize("M", [729, 32 * 729])
 def test_gelu_f16_epilogue(orc, weights, M):
     # fc1 with its output rounded to f16 for an F16 ffn_down: bit for bit
