@@ -32,7 +32,7 @@
 // Work decomposition.  128 x 128 output tiles, one per workgroup of 8 waves
 // (each 32 x 64: 2 subtiles), two workgroups per CU so that one's epilogue
 // and pipeline fill overlap the other's K loop.  GEMMs of too few such tiles
-// to give every CU two (batch 1, M = 729) run 64 x 128 tiles of 4 waves
+// to give every CU two (batch 1, M = 729) run smaller tiles of 1 to 4 waves
 // whose K stages are scheduled for a lone wave's latency instead.  The K
 // loop runs over stages of KS blocks whose operands (X and W quants and
 // scales) arrive by LDS DMA (buffer_load ... lds) into a ring of NS stage
@@ -70,23 +70,29 @@
 namespace s2x {
 namespace gemm {
 
-constexpr int BN = 128;  // output tile columns
+constexpr int BN_MAX = 128;  // most output tile columns of a form
 constexpr int GM = 8;    // tile-row group of the tile order
 constexpr int RM_N_TILES = 12;  // at most this many column tiles: row-major tile order
 constexpr int BUF_DW3 = 0x00020000;  // buffer resource word 3: raw 32-bit dwords
 
-// BM x 128 tiles (BM 128, 64 or 32), waves of 32 TM x 32 TN outputs (BM /
-// 32 TM along M, 128 / 32 TN along N); stages of KS K blocks in a ring of NS stage buffers
-// (NS - 1 stages in flight).  Throughput form (LAT false): as many
+// BM x BN tiles, waves of 32 TM x 32 TN outputs (BM / 32 TM along M, BN / 32
+// TN along N); stages of KS K blocks in a ring of NS stage buffers (NS - 1
+// stages in flight).  Throughput form (LAT false): 128 x 128, as many
 // workgroups per CU as two rings allow, each K block its own scheduling
 // region, <= 128 VGPRs (4 waves per SIMD cover each other's latency).
 // Latency form (LAT true, for GEMMs of too few tiles to give a SIMD more
-// than one or two waves): a stage's KS blocks are one scheduling region --
-// all their fragments read up front, their MFMAs interleaved -- with up to
-// 256 VGPRs, so that a lone wave keeps its matrix pipe busy.
-template <int KS_, int NS_, int BM_ = 128, bool LAT_ = false, int TM_ = 1, int TN_ = 2>
+// than one or two waves): the K loop pipelined over blocks and stages with
+// an imposed instruction order and up to 256 VGPRs.  What bounds it is the
+// lone wave's own issue, not the matrix pipe: three MFMAs and 16 fmas alone
+// take it 97 cycles a block (the pipe's 96), with a block's two quant and
+// two scale reads, their waits and masks 243.  Hence scale words read for two
+// blocks at a time, fragments read up to two blocks ahead over the stage's
+// barrier, no accumulator splat and DMA instructions one behind an MFMA: K =
+// 4320, N = 1152, M = 729 21.8 -> 20.2 us, M = 1000 38.5 -> 26.4, M = 64 19.0
+// -> 16.4 (with the tile forms below).
+template <int KS_, int NS_, int BM_ = 128, bool LAT_ = false, int TM_ = 1, int TN_ = 2, int BN_ = BN_MAX>
 struct Cfg {
-    static constexpr int TM = TM_, TN = TN_, BM = BM_, KS = KS_, NS = NS_;
+    static constexpr int TM = TM_, TN = TN_, BM = BM_, BN = BN_, KS = KS_, NS = NS_;
     static constexpr bool LAT = LAT_;
     // waves of 32 TM x 32 TN outputs, WN of them along N
     static constexpr int WN = BN / (32 * TN), NWAVE = BM / (32 * TM) * WN, NT = NWAVE * WAVE;
@@ -96,8 +102,10 @@ struct Cfg {
     // DMA instruction writes (rows past a 32-row tile are never read)
     static constexpr int XS_ROWS = BM < 64 ? 64 : BM;
     static constexpr int XS = WQ + KS * BN * 32;
-    static constexpr int WS = XS + KS * XS_ROWS * 4;  // [KS][BN] fp16 W scales
-    static constexpr int STAGE = WS + KS * BN * 2;
+    // [KS][WSC] fp16 W scales, whole groups of 64 columns; one instruction
+    // of 64 lanes writes them, 1,024 bytes whatever WSC
+    static constexpr int WS = XS + KS * XS_ROWS * 4, WSC = BN < 64 ? 64 : BN, WSL = WSC / 8;
+    static constexpr int STAGE = WS + 1024;
     static constexpr int LDS_BYTES = NS * STAGE;
     static constexpr int WG_PER_CU = 2 * LDS_BYTES <= 163840 ? 2 : 1;
     static constexpr int WPE = LAT ? 2 : WG_PER_CU * NWAVE / 4;  // waves per SIMD
@@ -112,10 +120,11 @@ struct Cfg {
     static constexpr int QPX = BM / 8 / NWAVE, QPW = BN / 8 / NWAVE;
     static_assert(KS == 4, "stage of 4 blocks: one 16-byte ds row per X row");
     static_assert(BM == 128 || BM == 64 || (BM == 32 && LAT && TN == 1), "tile rows");
+    static_assert(BN == BN_MAX || (LAT && TN == 1 && (BN == 64 || BN == 32)), "tile columns");
     static_assert(QPX >= 1 && QPW >= 1 && QPX * NWAVE * 8 == BM && QPW * NWAVE * 8 == BN, "DMA split");
     static_assert(STAGE % 128 == 0 && WQ % 128 == 0, "quant rows: chunk positions by xor");
     static_assert(NS == 2 || (LAT && NS <= 4), "ring: two stages, or up to four in the latency form");
-    static_assert(NSX + 1 <= NWAVE, "scale DMA waves");
+    static_assert(NSX + 1 <= NWAVE || NWAVE == 1, "scale DMA waves");
     static_assert(LDS_BYTES * WG_PER_CU <= 163840, "LDS");
     static_assert(NWAVE * 5120 <= LDS_BYTES, "epilogue scratch");
 };
@@ -538,6 +547,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     constexpr int TN = C::TN;
     const int wm = wave / C::WN, wn = wave % C::WN;
     const int lr = lane & 31, lh = lane >> 5;
+    constexpr int BN = C::BN;
     const int m_tiles = (M + BM - 1) / BM, n_tiles = (N + BN - 1) / BN;
     int tm, tn;
     tile_of(xcd_linear(blockIdx.x, gridDim.x), m_tiles, n_tiles, tm, tn);
@@ -559,7 +569,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     //   W quants, instructions t < QPW: likewise with QPW
     //   X scales: waves w < NSX, rows 64 w + lane, the ds words of blocks
     //             k0 .. k0 + 3 (16 bytes)
-    //   W scales: wave NSX, block lane / 16, columns 8 (lane % 16) .. + 7
+    //   W scales: wave NSX (a lone wave brings both), block lane / WSL,
+    //             columns 8 (lane % WSL) .. + 7 of the tile's 64-column groups
     uint32_t vqx[C::QPX], vqw[C::QPW], vxs, vws;
     {
         // chunk at position p of row r: p ^ swz8(r); in a GEMM of fewer than
@@ -574,7 +585,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 #pragma unroll
         for (int t = 0; t < C::QPW; ++t) vqw[t] = quant_off(8 * (C::QPW * wave + t) + (lane >> 3), ldw);
         vxs = (uint32_t)((min(wave, C::NSX - 1) * 64 + lane) * ld_ds * 4);
-        vws = (uint32_t)((lane >> 4) * ldT * 2 + (lane & 15) * 16);
+        vws = lane < KS * C::WSL ? (uint32_t)((lane / C::WSL) * ldT * 2 + (lane % C::WSL) * 16) : OOB_OFF;
     }
     // (the bases start at block kbs; the ranges end where the planes end)
     const __amdgpu_buffer_rsrc_t xr_live = __builtin_amdgcn_make_buffer_rsrc(
@@ -587,8 +598,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         (void *)(xds + (int64_t)m0 * ld_ds + kbs), (short)0,
         clip32((int64_t)(M - m0) * ld_ds * 4 - kbs * 4), BUF_DW3);
     const __amdgpu_buffer_rsrc_t wsr_live = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(wdT + (int64_t)kbs * ldT + n0), (short)0,
-        clip32(((int64_t)(KB_all - kbs) * ldT - n0) * 2), BUF_DW3);
+        (void *)(wdT + (int64_t)kbs * ldT + (n0 & ~63)), (short)0,
+        clip32(((int64_t)(KB_all - kbs) * ldT - (n0 & ~63)) * 2), BUF_DW3);
     const __amdgpu_buffer_rsrc_t none = __builtin_amdgcn_make_buffer_rsrc((void *)xq, (short)0, 0, BUF_DW3);
 
     // Issue the DMA of stage g into buffer g % NS.  Rows past M or N return
@@ -601,7 +612,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // stage buffer (shift = kb0 - kpos); a GEMM of fewer than KS blocks has
     // one partial stage, fetched by the first issue (outside the K loop)
     // with out-of-range lanes for the missing blocks and scales.  ROLE (a constant per wave: 1 X scales, 2 W
-    // scales, 0 neither) is a template value, so that no branch splits the
+    // scales, 3 both, 0 neither) is a template value, so that no branch splits the
     // K loop.
     // PART: 0 the X quants, 1 the W quants, 2 the scales, -1 all three
     auto kpos = [&](int g) { return KB >= KS ? min(g * KS, KB - KS) : g * KS; };
@@ -616,7 +627,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 for (int t = 0; t < C::QPX; ++t) dma16(xr_live, vqx[t], 0, sb + XQ + (C::QPX * wave + t) * 1024);
 #pragma unroll
                 for (int t = 0; t < C::QPW; ++t) dma16(wr_live, vqw[t], 0, sb + WQ + (C::QPW * wave + t) * 1024);
-                if constexpr (ROLE == 1) {
+                if constexpr (ROLE & 1) {
                     // one 4-byte DMA per ds word: 16 rows x KS words per
                     // instruction, the words of missing blocks out of range
 #pragma unroll
@@ -625,9 +636,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                         const uint32_t off = w < KB ? (uint32_t)((row * ld_ds + w) * 4) : OOB_OFF;
                         dma4(xsr_live, off, sb + XS + (64 * wave + 16 * t) * 16);
                     }
-                } else if constexpr (ROLE == 2) {
-                    dma16(wsr_live, (lane >> 4) < KB ? vws : OOB_OFF, 0, sb + WS);  // lane: block lane / 16
                 }
+                if constexpr (ROLE & 2) dma16(wsr_live, lane / C::WSL < KB ? vws : OOB_OFF, 0, sb + WS);
                 return;
             }
         }
@@ -643,13 +653,27 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             for (int t = 0; t < C::QPW; ++t) dma16(wr, vqw[t], k0 * 32, sb + WQ + (C::QPW * wave + t) * 1024);
         }
         if constexpr (PART == 2 || PART < 0) {
-            if constexpr (ROLE == 1)
-                dma16(xsr, vxs, k0 * 4, sb + XS + wave * 64 * 16);
-            else if constexpr (ROLE == 2)
-                dma16(wsr, vws, (uint32_t)(k0 * ldT * 2), sb + WS);
+            if constexpr (ROLE & 1) dma16(xsr, vxs, k0 * 4, sb + XS + wave * 64 * 16);
+            if constexpr (ROLE & 2) dma16(wsr, vws, (uint32_t)(k0 * ldT * 2), sb + WS);
         }
     };
     using All = std::integral_constant<int, -1>;
+    // instruction t of the stage's QPX + QPW (+ 1 scale) ones of this wave
+    auto issue_one = [&](int g, auto role, auto tc) {
+        constexpr int ROLE = decltype(role)::value, t = decltype(tc)::value;
+        const bool live = g < n_st;
+        uint8_t *sb = lds + (g % NS) * STAGE;
+        const uint32_t k0 = (uint32_t)kpos(g);
+        if constexpr (t < C::QPX) {
+            dma16(live ? xr_live : none, vqx[t], k0 * 32, sb + XQ + (C::QPX * wave + t) * 1024);
+        } else if constexpr (t < C::QPX + C::QPW) {
+            dma16(live ? wr_live : none, vqw[t - C::QPX], k0 * 32, sb + WQ + (C::QPW * wave + t - C::QPX) * 1024);
+        } else if constexpr (t == C::QPX + C::QPW && (ROLE & 1)) {
+            dma16(live ? xsr_live : none, vxs, k0 * 4, sb + XS + wave * 64 * 16);
+        } else {
+            dma16(live ? wsr_live : none, vws, (uint32_t)(k0 * ldT * 2), sb + WS);
+        }
+    };
 
     // Stage g + 1 visible to every wave: this wave's DMA of it has landed,
     // then the barrier.  After it no wave reads stage g's buffer any more, so
@@ -670,20 +694,23 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // X ds word (the scale d), both masked to zero on lanes 32..63 (k slots
     // 4..7); a 32 x 32 wave takes the half of the word its columns are
     const int sw_off = WS + (wn * TN / 2) * 128 + lr * 4;
-    const int sw_sh = TN == 1 ? 16 * (wn & 1) : 0;
+    const int sw_sh = TN == 1 ? 16 * ((n0 / 32 + wn) & 1) : 0;
     const uint32_t xmask = lh ? 0u : 0xffffu, wmask = lh ? 0u : ~0u;
     // slot j of the stage buffer (a constant in the K loop; the last
     // stage's block j + its window shift)
-    auto load_frag = [&](const uint8_t *sb, int j, Frag<TM, TN> &f) {
+    auto load_quants = [&](const uint8_t *sb, int j, Frag<TM, TN> &f) {
 #pragma unroll
         for (int a = 0; a < TM; ++a)
             f.a[a] = *reinterpret_cast<const v4i *>(sb + (a_off ^ (j * 32)) + a * 32 * 128);
 #pragma unroll
         for (int b = 0; b < TN; ++b)
             f.b[b] = *reinterpret_cast<const v4i *>(sb + (b_off ^ (j * 32)) + b * 32 * 128);
+    };
+    auto load_frag = [&](const uint8_t *sb, int j, Frag<TM, TN> &f) {
+        load_quants(sb, j, f);
 #pragma unroll
         for (int a = 0; a < TM; ++a) f.xw[a] = *reinterpret_cast<const uint32_t *>(sb + sx_off + j * 4 + a * 32 * 16);
-        f.wp = *reinterpret_cast<const uint32_t *>(sb + sw_off + j * BN * 2);
+        f.wp = *reinterpret_cast<const uint32_t *>(sb + sw_off + j * C::WSC * 2);
     };
     // the scale operands of subtile (a, b), from the raw words: the VALU
     // work sits with the MFMAs that use it, not with the (early) reads
@@ -792,47 +819,89 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
 
     // Latency form, software-pipelined over K blocks (each output's fma
     // chain is the only serial dependency; a block's MFMAs depend on
-    // nothing of the block before).  Slot j of a stage: read block j + 1's
-    // fragments, issue block j's MFMAs (block dots, scale tiles, then the
-    // conversions, into ring entry j % 2) and run block j - 1's fmas from
-    // ring entry (j - 1) % 2, one MFMA per five VALU instructions, so that
-    // the wave's matrix pipe and VALU work side by side.  Block 3's fmas
-    // run in slot 0 of the next stage (after its barrier); the fmas stay in
-    // block order.
-    struct Ring {
-        v16f I[NSUB], S[NSUB];
-    };
-    auto mfma_group = [&](const Frag<TM, TN> &f, Ring &R) {
-        v16i D[NSUB];
-        const v16f zf = {};
-        const v16i magic = 0x3E22F983;
+    // nothing of the block before).  A lone wave has nothing but its own
+    // instruction order to keep its matrix pipe busy, so the order is
+    // imposed MFMA by MFMA.  Slot j of a stage: read the fragments of block
+    // j + PD (over the stage's end: the next stage's), then the 3 NSUB
+    // MFMAs of block j (block dots, scale tiles, conversions, into ring
+    // entry j % 2), behind each of them a share of the stage's DMA
+    // instructions and of the earlier block's fmas, which start LAG MFMAs
+    // into the slot: a conversion's result is read two MFMAs after it, when
+    // it is there.  The fmas stay in block order.
+    constexpr int NMF = 3 * NSUB, LAG = NSUB == 1 ? 1 : 0;
+    // fragments PD blocks ahead: two slots cover the LDS latency where the
+    // registers allow it
+    constexpr int PD = NSUB == 1 ? 2 : 1, NF = 2 * PD;
+    // block j's dots, converted in place, in entry j % NI, its scale tiles in
+    // entry j % 2 (with LAG the dots of block j are issued while block j -
+    // 2's are still read)
+    constexpr int NI = NSUB == 1 ? 4 : 2;
+    v16f RI[NI][NSUB], RS[2][NSUB];
+    // share c of NMF of block j's fmas
+    auto fma_share = [&](auto jc, auto cc) {
+        constexpr int j = decltype(jc)::value;
+        constexpr int c = decltype(cc)::value, lo = 16 * NSUB * c / NMF, hi = 16 * NSUB * (c + 1) / NMF;
 #pragma unroll
-        for (int k = 0; k < NSUB; ++k)
-            D[k] = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[k / TN], f.b[k % TN], magic, 0, 0, 0);
-#pragma unroll
-        for (int k = 0; k < NSUB; ++k)
-            R.S[k] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, sx_op(f, k / TN)),
-                                                          __builtin_bit_cast(v4h, sw_op(f, k % TN)), zf, 0, 0, 0);
-#pragma unroll
-        for (int k = 0; k < NSUB; ++k)
-            R.I[k] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, cA), __builtin_bit_cast(v4h, cB),
-                                                          __builtin_bit_cast(v16f, D[k]), 0, 0, 0);
-    };
-    auto fma_group = [&](const Ring &R) {
-#pragma unroll
-        for (int k = 0; k < NSUB; ++k)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                acc[k / TN][k % TN][r] = fmaf(R.I[k][r], R.S[k][r], acc[k / TN][k % TN][r]);
-    };
-    // the slot's order: fragment reads first, then MFMA / VALU alternating
-    auto slot_order = [&]() {
-        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-#pragma unroll
-        for (int i = 0; i < 3 * NSUB; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        for (int i = lo; i < hi; ++i) {
+            const int k = i / 16, r = i % 16;
+            acc[k / TN][k % TN][r] = fmaf(RI[j % NI][k][r], RS[j & 1][k][r], acc[k / TN][k % TN][r]);
         }
+    };
+    // raw scale words of a stage's blocks: read a pair of blocks at a time
+    struct Scales {
+        uint32_t xw[KS][TM], wp[KS];
+    } sc;
+    auto load_scales = [&](const uint8_t *sb, int j0, auto jc, auto nc) {
+        constexpr int j = decltype(jc)::value, n = decltype(nc)::value;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+#pragma unroll
+            for (int a = 0; a < TM; ++a)
+                sc.xw[j + i][a] = *reinterpret_cast<const uint32_t *>(sb + sx_off + (j0 + i) * 4 + a * 32 * 16);
+            sc.wp[j + i] = *reinterpret_cast<const uint32_t *>(sb + sw_off + (j0 + i) * C::WSC * 2);
+        }
+    };
+    using std::integral_constant;
+    // the MFMAs of block j (f: its fragments), the rest of block j - 2's fmas
+    // and most of block j - 1's; dma(c): share c of NMF of the slot's DMA
+    // instructions
+    auto slot = [&](Frag<TM, TN> &f, auto jc, auto in_loop, auto &&dma) {
+        constexpr int j = decltype(jc)::value;
+#pragma unroll
+        for (int a = 0; a < TM; ++a) f.xw[a] = sc.xw[j][a];
+        f.wp = sc.wp[j];
+        static_for<NMF>([&](auto ic) {
+            constexpr int i = decltype(ic)::value, k = i % NSUB;
+            v16f &I = RI[j % NI][k];
+            dma(ic);
+            if constexpr (i < NSUB) {
+                if constexpr (decltype(in_loop)::value) {
+                    // the accumulator as the inline constant 1/2pi, as in
+                    // the throughput form (a splat that several MFMAs use is
+                    // built anew in 16 VGPRs every stage); the result's one
+                    // reader is the conversion below, in place
+                    asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0.15915494"
+                                 : "=&v"(I)
+                                 : "v"(f.a[k / TN]), "v"(f.b[k % TN]));
+                } else {
+                    // around the loop, where the compiler may copy the
+                    // result, by the builtin, whose hazards it knows
+                    const v16i magic = 0x3E22F983;
+                    I = __builtin_bit_cast(v16f, __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[k / TN], f.b[k % TN], magic, 0, 0, 0));
+                }
+            } else if constexpr (i < 2 * NSUB) {
+                const v16f zf = {};
+                RS[j & 1][k] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, sx_op(f, k / TN)),
+                                                                    __builtin_bit_cast(v4h, sw_op(f, k % TN)), zf, 0, 0, 0);
+            } else {
+                I = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, cA), __builtin_bit_cast(v4h, cB), I, 0, 0, 0);
+            }
+            if constexpr (i < LAG)
+                fma_share(integral_constant<int, (j + KS - 2) % KS>{}, integral_constant<int, i - LAG + NMF>{});
+            else
+                fma_share(integral_constant<int, (j + KS - 1) % KS>{}, integral_constant<int, i - LAG>{});
+            __builtin_amdgcn_sched_barrier(0);
+        });
     };
     // NS - 1 stages in flight: the DMA instructions this wave issues per
     // stage (a constant of its role), so that the wait for a stage lets
@@ -840,48 +909,90 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // order)
     auto k_loop_pipelined = [&](auto role) {
         constexpr int ROLE = decltype(role)::value;
-        constexpr int DPS = C::QPX + C::QPW + (ROLE != 0 ? 1 : 0);
+        constexpr int DPS = C::QPX + C::QPW + (ROLE & 1) + (ROLE >> 1);
         issue(0, role, All{}, std::true_type{});
         static_for<NS - 1>([&](auto sc) { issue(1 + decltype(sc)::value, role, All{}, std::false_type{}); });
         wait_vm<(NS - 1) * DPS>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        // ring entry 1 starts at zero: the first stage's slot 0 runs its
-        // fmas as fmaf(0, 0, acc) = acc (acc is never -0)
-        Ring R[2];
+        // the rings start at zero: the first slots' fmas of blocks -1 and -2
+        // are fmaf(0, 0, acc) = acc (acc is never -0)
 #pragma unroll
-        for (int k = 0; k < NSUB; ++k) R[1].I[k] = R[1].S[k] = v16f{};
-        Frag<TM, TN> Fs[2];
-        // every stage but the last: KS blocks, no branch
-        for (int g = 0; g < n_st - 1; ++g) {
-            const uint8_t *sb = lds + (g % NS) * STAGE;
-            load_frag(sb, 0, Fs[0]);
-            static_for<KS>([&](auto jc) {
-                constexpr int j = decltype(jc)::value;
-                if constexpr (j + 1 < KS) load_frag(sb, j + 1, Fs[(j + 1) & 1]);
-                mfma_group(Fs[j & 1], R[j & 1]);
-                fma_group(R[(j + 1) & 1]);  // block j - 1 (slot 0: the previous stage's block 3)
-                slot_order();
-                __builtin_amdgcn_sched_barrier(0);
-            });
-            // stage g + 1 landed (stages g + 2 .. g + NS - 1 may still be
-            // in flight), every wave past stage g: its buffer takes stage
-            // g + NS
+        for (int k = 0; k < NSUB; ++k) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) RI[i][k] = v16f{};
+            RS[0][k] = RS[1][k] = v16f{};
+        }
+        Frag<TM, TN> Fs[NF];
+        const auto no_dma = [](auto) {};
+        // the last stage: nb = 1 .. KS blocks, block kb0 + j in slot
+        // j + shift of its buffer (a partial stage was fetched as the window
+        // of the last KS blocks)
+        const uint8_t *sbl = lds + ((n_st - 1) % NS) * STAGE;
+        const int nb = KB - (n_st - 1) * KS, shift = (n_st - 1) * KS - kpos(n_st - 1);
+        // stage g + 1 landed (stages g + 2 .. g + NS - 1 may still be in
+        // flight) and every wave has read its last fragments of stage g,
+        // whose buffer takes stage g + NS from here on
+        auto next_stage = [&]() {
             wait_vm<(NS - 2) * DPS>();
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            issue(g + NS, role, All{}, std::false_type{});
+        };
+        if (n_st > 1) {
+            load_scales(lds, 0, integral_constant<int, 0>{}, integral_constant<int, KS>{});
+            static_for<PD>([&](auto jc) { load_quants(lds, decltype(jc)::value, Fs[decltype(jc)::value]); });
+            static_for<KS - PD>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                load_quants(lds, j + PD, Fs[(j + PD) % NF]);
+                slot(Fs[j % NF], jc, std::false_type{}, no_dma);
+            });
+            // stage g's last PD slots and stage g + 1's others, no branch
+            for (int g = 0; g < n_st - 2; ++g) {
+                next_stage();
+                const uint8_t *sb = lds + ((g + 1) % NS) * STAGE;
+                static_for<KS>([&](auto tc) {
+                    constexpr int t = decltype(tc)::value, j = (t + KS - PD) % KS;
+                    load_quants(sb, t, Fs[t % NF]);
+                    if constexpr (t % 2 == 0) load_scales(sb, t, tc, integral_constant<int, 2>{});
+                    slot(Fs[j % NF], integral_constant<int, j>{}, std::true_type{}, [&](auto ic) {
+                        constexpr int lo = DPS * (t * NMF + decltype(ic)::value) / (KS * NMF);
+                        constexpr int hi = DPS * (t * NMF + decltype(ic)::value + 1) / (KS * NMF);
+                        if constexpr (hi > lo) issue_one(g + NS, role, std::integral_constant<int, lo>{});
+                        static_assert(hi - lo <= 1, "at most one DMA instruction per MFMA");
+                    });
+                });
+            }
+            next_stage();
+            static_for<PD>([&](auto tc) {
+                constexpr int t = decltype(tc)::value, j = t + KS - PD;
+                load_quants(sbl, min(t + shift, KS - 1), Fs[t % NF]);
+                load_scales(sbl, min(t + shift, KS - 1), tc, integral_constant<int, 1>{});
+                slot(Fs[j % NF], integral_constant<int, j>{}, std::false_type{}, no_dma);
+            });
+        } else {
+            static_for<PD>([&](auto jc) {
+                load_quants(sbl, decltype(jc)::value, Fs[decltype(jc)::value]);
+                load_scales(sbl, decltype(jc)::value, jc, integral_constant<int, 1>{});
+            });
         }
-        // the last stage: the previous stage's block 3, then nb = 1 .. KS
-        // blocks one at a time, block kb0 + j in slot j + shift (a partial
-        // stage was fetched as the window of the last KS blocks)
-        fma_group(R[1]);
-        const uint8_t *sb = lds + ((n_st - 1) % NS) * STAGE;
-        const int kb0 = (n_st - 1) * KS, nb = KB - kb0, shift = kb0 - kpos(n_st - 1);
         static_for<KS>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
             if (j < nb) {
-                load_frag(sb, j + shift, Fs[0]);
-                mfma_group(Fs[0], R[0]);
-                fma_group(R[0]);
+                if constexpr (j + PD < KS) {
+                    const int p = min(j + PD + shift, KS - 1);
+                    load_quants(sbl, p, Fs[(j + PD) % NF]);
+                    load_scales(sbl, p, integral_constant<int, j + PD>{}, integral_constant<int, 1>{});
+                }
+                slot(Fs[j % NF], jc, std::false_type{}, no_dma);
+            }
+        });
+        // what is left: the block before the last one's last LAG shares, then
+        // the last one's (block l of the last stage)
+        static_for<KS>([&](auto lc) {
+            constexpr int l = decltype(lc)::value;
+            if (l == nb - 1) {
+                static_for<LAG>([&](auto cc) {
+                    fma_share(integral_constant<int, (l + KS - 1) % KS>{}, integral_constant<int, NMF - LAG + decltype(cc)::value>{});
+                });
+                static_for<NMF>([&](auto cc) { fma_share(lc, cc); });
             }
         });
     };
@@ -943,7 +1054,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         });
     }
     };
-    if (wave < C::NSX)
+    if constexpr (C::NWAVE == 1)
+        k_loop(std::integral_constant<int, 3>{});
+    else if (wave < C::NSX)
         k_loop(std::integral_constant<int, 1>{});
     else if (wave == C::NSX)
         k_loop(std::integral_constant<int, 2>{});
@@ -977,7 +1090,7 @@ hipError_t run(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_
         if (e != hipSuccess) return e;
         attr_set = true;
     }
-    const int64_t tiles = ((M + C::BM - 1) / C::BM) * ((w.N + BN - 1) / BN);
+    const int64_t tiles = ((M + C::BM - 1) / C::BM) * ((w.N + C::BN - 1) / C::BN);
     const int64_t KB = w.K_pad / QK;
     const unsigned splits = epi.kb_split > 0 ? (unsigned)((KB + epi.kb_split - 1) / epi.kb_split) : 1u;
     // without scales (the block-dot dump) the scale DMA reads a zero-size
@@ -1452,28 +1565,33 @@ static hipError_t run_gemv_epi(const WeightView &w, const int8_t *xq, const uint
 
 // Stage configurations: 4-block stages in a ring of 2.  Wide: 128 x 128
 // tiles, two workgroups per CU, for GEMMs of enough tiles to fill the chip.
-// Small: 64 x 128 tiles in the latency form, for GEMMs of fewer 128 x 128
-// tiles than two per CU (M = 729: batch 1).  Each output's K order is the
-// same in both, so the choice does not change a bit.  At M = 729 the small
-// form takes out from 19.8 to 14.6 us and fc2 from 58.7 to 42.5 us; rings
-// of 3 or 4 stages, 2-block stages and an imposed MFMA / VALU alternation
-// measured slower.
+// Small: the latency form, for GEMMs of fewer 128 x 128 tiles than two per
+// CU.  Each output's K order is the same in all, so the choice does not
+// change a bit (M = 729 in 128 x 128 tiles: out 19.8 us, fc2 58.7).
 #ifndef S2X_WIDE_TM
 #define S2X_WIDE_TM 1
 #endif
 using Wide = gemm::Cfg<4, 2, 128, false, S2X_WIDE_TM>;
 // The latency form's ring: four stages (three in flight) where its
-// workgroups fit one per CU, three stages (two per CU) otherwise.  Where
-// they fit one per CU, the plain / bias / residual epilogues (the out
-// projection and fc2) run 8 waves of 32 x 32 outputs per 64 x 128 tile
-// (Small4W): twice the waves, each with half the MFMA chain.  Where even
-// those tiles number fewer than the CUs (out and fc2 at M = 729: 108 of
-// them), 32 x 128 tiles of 4 such waves (Small4T) spread the rows over
-// twice the workgroups: the same per-output K order, without splitting K.
+// workgroups fit one per CU, three stages (two per CU) otherwise.  The plain
+// / bias / residual epilogues (the out projection, fc2, the text tower's
+// QKV) run waves of 32 x 32 outputs, in the smallest tiles that still give
+// every workgroup a CU of its own (a workgroup's DMA, about 40 bytes per ns
+// from past the L2, is what a smaller tile shortens): one wave (Lone), two
+// (Narrow), else 64 x 64 tiles of four while all are resident, two per CU
+// (Square: 16 KB of quants a stage where 32 x 128 tiles take 20).  K = 4320,
+// N = 1152: M = 64 Lone 16.4 us, Narrow 17.0, Square 17.5; M = 320 Narrow
+// 18.1 to 18.6, Lone 18.4, Square 18.7; M = 729 Square 20.2, 32 x 128 20.5,
+// Narrow 25.3, Lone 33.4.  K = 1152: M = 320, N = 3456 Square 10.4, Narrow
+// 13.9, 32 x 128 14.3; M = 1458, N = 1152 Square 11.6, 32 x 128 15.6.  More
+// than two Square workgroups per CU: 64 x 128 tiles of waves with two
+// subtiles (M = 1800: 43.1 us, 46.0 before).  The same per-output K order in
+// all, without splitting K.
 using Small4 = gemm::Cfg<4, 4, 64, true>;
-using Small4W = gemm::Cfg<4, 4, 64, true, 1, 1>;
-using Small4T = gemm::Cfg<4, 4, 32, true, 1, 1>;
 using Small3 = gemm::Cfg<4, 3, 64, true>;
+using Lone = gemm::Cfg<4, 4, 32, true, 1, 1, 32>;
+using Narrow = gemm::Cfg<4, 4, 32, true, 1, 1, 64>;
+using Square = gemm::Cfg<4, 4, 64, true, 1, 1, 64>;
 
 template <int E>
 static hipError_t run_small(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds,
@@ -1483,8 +1601,6 @@ static hipError_t run_small(const WeightView &w, const int8_t *xq, int64_t ldx, 
 static bool use_small(int64_t M, int64_t N) {
     return ((M + 127) / 128) * ((N + 127) / 128) < 2 * 256;
 }
-static bool small_ring4(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 127) / 128) <= 256; }
-static bool small_rows32(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 127) / 128) < 256; }
 
 hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xds, int64_t ld_ds,
                        int64_t M, float *y, int64_t ldy, const EpiParams &epi_in,
@@ -1499,7 +1615,7 @@ hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xd
         M > (1 << 30) || w.N > (1 << 30) || ((uintptr_t)xq & 15) || ((uintptr_t)w.qs & 15) ||
         ((uintptr_t)xds & 3) || (epi.kind != EPI_DUMP_I && (!xds || ld_ds < KB)) ||
         ldx < w.K_pad || ldx % 16 || w.ld_qs < w.K_pad || w.ld_qs % 16 || (int64_t)C::BM * ldx > 0x7fffffff ||
-        (int64_t)gemm::BN * w.ld_qs > 0x7fffffff || w.ldT * KB * 2 > 0x7fffffff ||
+        (int64_t)gemm::BN_MAX * w.ld_qs > 0x7fffffff || w.ldT * KB * 2 > 0x7fffffff ||
         C::BM * ld_ds * 4 > 0x7fffffff || C::BM * ldy * 4 > 0x7fffffff ||
         (epi.kb_split != 0 && (epi.kind != EPI_NONE || epi.kb_split < 0 || epi.y_split < M * ldy)))
         return hipErrorInvalidValue;
@@ -1546,12 +1662,15 @@ static hipError_t run_small(const WeightView &w, const int8_t *xq, int64_t ldx, 
                             hipStream_t stream) {
     constexpr bool plain = E == EPI_NONE || E == EPI_BIAS || E == EPI_BIAS_GELU || E == EPI_BIAS_RESID ||
                            E == EPI_DUMP_I;
-    if (!small_ring4(M, w.N)) return gemm::run<Small3, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+    const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((w.N + bn - 1) / bn); };
     if constexpr (plain) {
-        if (small_rows32(M, w.N)) return gemm::run<Small4T, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
-        return gemm::run<Small4W, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        if (tiles(32, 32) <= 256) return gemm::run<Lone, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        if (tiles(32, 64) <= 256) return gemm::run<Narrow, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        if (tiles(64, 64) <= 512) return gemm::run<Square, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+    } else {
+        if (tiles(64, 128) <= 256) return gemm::run<Small4, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
     }
-    return gemm::run<Small4, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+    return gemm::run<Small3, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
 }
 
 // The form of an F16 product, by tiles per round of the 256 CUs (every form

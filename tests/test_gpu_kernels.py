@@ -265,6 +265,29 @@ def test_gemm_short_k(orc, KB, form):
         s2x.lib.s2x_weight_destroy(w)
 
 
+@pytest.mark.parametrize("M,N", [(31, 65), (33, 1152), (300, 1003), (321, 1001), (700, 1003), (1400, 500)])
+@pytest.mark.parametrize("KB", [1, 3, 4, 5, 8, 11, 14])
+def test_gemm_latency_forms(orc, M, N, KB):
+    # 32 x 32, 32 x 64, 64 x 64 and 64 x 128 tiles at ragged edges, around
+    # whole and partial stages of 4 blocks; the sums are the oracle's bits
+    K = 32 * KB
+    say(f"gemm latency form: KB={KB} M={M} N={N}")
+    rng = np.random.default_rng(90 + KB)
+    raw = synth.quantize_q8_0(rng.normal(0, 0.02, (N, K)).astype(np.float32), K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    qs, ds = _quant_gpu(x, K)
+    rows = np.arange(M) if M < 100 else np.unique(np.concatenate([rng.choice(M, 60, replace=False), np.arange(M - 40, M)]))
+    rq, rd = orc.quantize_q8_1(x[rows], K)
+    ref = orc.mul_mat_q8_0_q8_1(raw, K, N, rq, rd)
+    w = _weight(raw, K, N)
+    try:
+        y = empty((M, N), torch.float32)
+        s2x.call("s2x_mul_mat_q8_0_q8_1", w, ptr(qs), ptr(ds), M, ptr(y), N, None, stream())
+        assert_same(host(y)[rows], ref, f"gemm KB={KB} M={M} N={N}")
+    finally:
+        s2x.lib.s2x_weight_destroy(w)
+
+
 def test_gemm_large_m_batch_invariant(orc, gemm_data):
     raw, N, K, K_pad = gemm_data["fc2"]
     M = 23328
