@@ -10,6 +10,7 @@
 
 #include "s2x_device.h"
 #include "s2x_kernels.h"
+#include "s2x_plan.h"
 
 #include <type_traits>
 
@@ -127,22 +128,25 @@ hipError_t launch_repack_q8_0(const void *raw, int64_t K_pad, int64_t N, int8_t 
 // f16 rows of ldx16 halves (round to nearest even, as ggml's F32 -> F16 of
 // the vec_dot operand), and, where the raw weight cannot be read in place,
 // its rows of K halves -> rows of ldw halves; zeros past K.  Both only move
-// bytes.  A block takes 4 rows x 512 columns, a lane 8 halves: 32-byte reads
-// of x, 16-byte stores, and one (wave-uniform) division per block.
-// 2,916 rows of K = 4,304: 12.1 us, 6.2 TB/s (64-bit divisions per 4 halves
-// and 4-byte loads before).
+// bytes.  A lane takes 8 halves of a row (32-byte reads of x, 16-byte
+// stores), a block as many rows as f16_operand_grid says, with one
+// (wave-uniform) division.  2,916 rows of K = 4,304: 12.1 us, 6.2 TB/s
+// (64-bit divisions per 4 halves and 4-byte loads before).
 // ---------------------------------------------------------------------------
 template <bool VEC>
 __global__ __launch_bounds__(256) void k_f16_operands(const float *__restrict__ x, int64_t K, int64_t M,
                                                       int64_t ldx, _Float16 *__restrict__ x16, int64_t ldx16,
-                                                      unsigned x_blocks, const uint16_t *__restrict__ raw,
-                                                      int64_t N, uint16_t *__restrict__ w16, int64_t ldw) {
+                                                      unsigned x_blocks, int x_lg, unsigned x_ncb,
+                                                      const uint16_t *__restrict__ raw, int64_t N,
+                                                      uint16_t *__restrict__ w16, int64_t ldw, int w_lg,
+                                                      unsigned w_ncb) {
     const bool is_x = blockIdx.x < x_blocks;
     const unsigned bid = is_x ? blockIdx.x : blockIdx.x - x_blocks;
-    const unsigned ncb = (unsigned)(((is_x ? ldx16 : ldw) + 511) / 512);
+    const unsigned ncb = is_x ? x_ncb : w_ncb;
+    const int lg = is_x ? x_lg : w_lg;
     const unsigned rg = bid / ncb;
-    const int64_t row = (int64_t)rg * 4 + (threadIdx.x >> 6);
-    const int64_t c = (int64_t)(bid - rg * ncb) * 512 + (threadIdx.x & 63) * 8;
+    const int64_t row = (int64_t)rg * (256 >> lg) + (threadIdx.x >> lg);
+    const int64_t c = ((int64_t)(bid - rg * ncb) << (lg + 3)) + (threadIdx.x & ((1u << lg) - 1)) * 8;
     if (is_x) {
         if (row >= M || c >= ldx16) return;
         const float *r = x + row * ldx;
@@ -171,12 +175,13 @@ hipError_t launch_f16_operands(const float *x, int64_t K, int64_t M, int64_t ldx
                                const void *raw, int64_t N, _Float16 *w16, int64_t ldw, hipStream_t stream) {
     if (M == 0) return hipSuccess;
     if (ldx16 % 8 || ldx16 < K || (raw && (ldw % 8 || ldw < K))) return hipErrorInvalidValue;
-    const int64_t xb = (M + 3) / 4 * ((ldx16 + 511) / 512), wb = raw ? (N + 3) / 4 * ((ldw + 511) / 512) : 0;
-    if (xb + wb > 0x7fffffff) return hipErrorInvalidValue;
+    const F16OperandGrid gx = f16_operand_grid(M, ldx16), gw = f16_operand_grid(raw ? N : 0, raw ? ldw : 8);
+    if ((gx.blocks + gw.blocks) * 256 > GRID_MAX_THREADS) return hipErrorInvalidValue;
     const bool vec = ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-    hipLaunchKernelGGL(vec ? k_f16_operands<true> : k_f16_operands<false>, dim3((unsigned)(xb + wb)), dim3(256), 0,
-                       stream, x, K, M, ldx, x16, ldx16, (unsigned)xb, reinterpret_cast<const uint16_t *>(raw), N,
-                       reinterpret_cast<uint16_t *>(w16), ldw);
+    hipLaunchKernelGGL(vec ? k_f16_operands<true> : k_f16_operands<false>, dim3((unsigned)(gx.blocks + gw.blocks)),
+                       dim3(256), 0, stream, x, K, M, ldx, x16, ldx16, (unsigned)gx.blocks, gx.lg_lanes,
+                       (unsigned)gx.col_blocks, reinterpret_cast<const uint16_t *>(raw), N,
+                       reinterpret_cast<uint16_t *>(w16), ldw, gw.lg_lanes, (unsigned)gw.col_blocks);
     return hipGetLastError();
 }
 

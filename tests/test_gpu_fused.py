@@ -425,6 +425,24 @@ def test_mul_mat_f16_forms(M, K, N, off):
     assert (np.abs(host(y) - ref) <= K * 2.0 ** -24 * _f16_terms_abs(w16, x)).all()
 
 
+def test_mul_mat_f16_many_rows():
+    # more rows than one wave each allows a launch (2^32 threads)
+    M, K, N = (1 << 26) + 3, 8, 1
+    say(f"F16 mul_mat M={M} K={K} N={N}")
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(58)
+    xd = torch.randn(M, K, generator=g, device="cuda:0")
+    wd = torch.randn(N, K, generator=g, device="cuda:0").to(torch.float16)
+    wsb = s2x.lib.s2x_mul_mat_f16_workspace_size(K, N, M)
+    ws, y = empty((wsb,), torch.uint8), torch.full((M, N), float("nan"), device="cuda:0")
+    s2x.call("s2x_mul_mat_f16_f32", ptr(wd), K, N, ptr(xd), K, M, ptr(y), ptr(ws), ctypes.c_size_t(wsb), stream())
+    torch.cuda.synchronize()
+    xh, w = xd.to(torch.float16).double(), wd.double()
+    ref, terms = (xh * w).sum(1), (xh.abs() * w.abs()).sum(1)
+    # K f32 additions of exact products, in any order
+    assert bool(((y[:, 0].double() - ref).abs() <= K * 2.0 ** -24 * terms).all())
+
+
 @pytest.mark.parametrize("M", [729, 32 * 729])
 def test_gelu_f16_epilogue(orc, weights, M):
     # fc1 with its output rounded to f16 for an F16 ffn_down: bit for bit

@@ -1,0 +1,56 @@
+"""The rules by which the launchers choose grids and layouts from sizes
+(csrc/s2x_plan.h), compiled for the CPU."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "hbd-siglip2.cpp_amd", "csrc")
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    so = tmp_path_factory.mktemp("plan") / "launch_plan.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", CSRC, "-o", str(so),
+                    os.path.join(HERE, "cpp", "launch_plan.cpp")], check=True)
+    return ctypes.CDLL(str(so))
+
+
+def _operand_grid(plan, rows, ld):
+    out = (ctypes.c_int64 * 3)()
+    plan.plan_f16_operand_grid(ctypes.c_int64(rows), ctypes.c_int64(ld), out)
+    return tuple(out)  # log2 of the lanes per row, blocks along a row, blocks
+
+
+def _up(a, b):
+    return (a + b - 1) // b * b
+
+
+@pytest.mark.parametrize("rows", [1, 3, 4, 63, 64, 65, 257])
+@pytest.mark.parametrize("ld", [8, 16, 24, 32, 64, 72, 256, 264, 512, 520, 544, 1024, 4352])
+def test_f16_operand_grid_covers_each_chunk_once(plan, rows, ld):
+    lg, ncb, blocks = _operand_grid(plan, rows, ld)
+    bid, tid = np.divmod(np.arange(blocks * 256), 256)
+    row = bid // ncb * (256 >> lg) + (tid >> lg)
+    c = (bid % ncb) * (8 << lg) + (tid & ((1 << lg) - 1)) * 8
+    ok = (row < rows) & (c < ld)
+    assert np.array_equal(np.unique(row[ok] * ld + c[ok]), np.arange(0, rows * ld, 8))
+    assert ok.sum() == rows * ld // 8
+
+
+def test_f16_operand_grid_takes_rows_up_to_the_launch_limit(plan):
+    # HIP refuses 2^32 threads along x.  A thread per 4 halves of rows padded
+    # to 32 stays below that up to 2^34 / K_pad rows; the grid must take all
+    # of those, at the stride of whole 128-byte lines too (2^26 rows of K = 8
+    # among them, where 64 lanes a row are 2^32 threads)
+    for K in (*range(8, 2200, 8), 4304, 65536, 1 << 20):
+        k_pad = _up(K, 32)
+        rows = min(1 << 30, ((1 << 32) - 256) * 4 // k_pad)
+        for ld in (k_pad, _up(K, 64)):
+            assert _operand_grid(plan, rows, ld)[2] * 256 < 1 << 32, (K, ld, rows)
