@@ -133,7 +133,12 @@ hipError_t launch_repack_q8_0(const void *raw, int64_t K_pad, int64_t N, int8_t 
 // (wave-uniform) division.  2,916 rows of K = 4,304: 12.1 us, 6.2 TB/s
 // (64-bit divisions per 4 halves and 4-byte loads before).
 // ---------------------------------------------------------------------------
-template <bool VEC>
+// 4 floats of a row at any 4-byte boundary: the vector memory path takes
+// 16-byte loads at dword addresses, so odd row strides need no path of their
+// own (with 8 dword loads a lane, 32 bytes apart, 23,328 rows of K = 1,001
+// took 139 us with their GEMM of N = 1,152, now 89)
+typedef v4f v4f_dw __attribute__((aligned(4)));
+
 __global__ __launch_bounds__(256) void k_f16_operands(const float *__restrict__ x, int64_t K, int64_t M,
                                                       int64_t ldx, _Float16 *__restrict__ x16, int64_t ldx16,
                                                       unsigned x_blocks, int x_lg, unsigned x_ncb,
@@ -151,11 +156,11 @@ __global__ __launch_bounds__(256) void k_f16_operands(const float *__restrict__ 
         if (row >= M || c >= ldx16) return;
         const float *r = x + row * ldx;
         _Float16 v[8];
-        if (VEC && c + 8 <= K) {
-            const float4 t0 = *reinterpret_cast<const float4 *>(r + c);
-            const float4 t1 = *reinterpret_cast<const float4 *>(r + c + 4);
-            v[0] = f32_to_f16(t0.x); v[1] = f32_to_f16(t0.y); v[2] = f32_to_f16(t0.z); v[3] = f32_to_f16(t0.w);
-            v[4] = f32_to_f16(t1.x); v[5] = f32_to_f16(t1.y); v[6] = f32_to_f16(t1.z); v[7] = f32_to_f16(t1.w);
+        if (c + 8 <= K) {
+            const v4f t0 = *reinterpret_cast<const v4f_dw *>(r + c);
+            const v4f t1 = *reinterpret_cast<const v4f_dw *>(r + c + 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = f32_to_f16(t0[j]), v[4 + j] = f32_to_f16(t1[j]);
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = c + j < K ? f32_to_f16(r[c + j]) : (_Float16)0.0f;
@@ -177,11 +182,10 @@ hipError_t launch_f16_operands(const float *x, int64_t K, int64_t M, int64_t ldx
     if (ldx16 % 8 || ldx16 < K || (raw && (ldw % 8 || ldw < K))) return hipErrorInvalidValue;
     const F16OperandGrid gx = f16_operand_grid(M, ldx16), gw = f16_operand_grid(raw ? N : 0, raw ? ldw : 8);
     if ((gx.blocks + gw.blocks) * 256 > GRID_MAX_THREADS) return hipErrorInvalidValue;
-    const bool vec = ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-    hipLaunchKernelGGL(vec ? k_f16_operands<true> : k_f16_operands<false>, dim3((unsigned)(gx.blocks + gw.blocks)),
-                       dim3(256), 0, stream, x, K, M, ldx, x16, ldx16, (unsigned)gx.blocks, gx.lg_lanes,
-                       (unsigned)gx.col_blocks, reinterpret_cast<const uint16_t *>(raw), N,
-                       reinterpret_cast<uint16_t *>(w16), ldw, gw.lg_lanes, (unsigned)gw.col_blocks);
+    hipLaunchKernelGGL(k_f16_operands, dim3((unsigned)(gx.blocks + gw.blocks)), dim3(256), 0, stream, x, K, M, ldx,
+                       x16, ldx16, (unsigned)gx.blocks, gx.lg_lanes, (unsigned)gx.col_blocks,
+                       reinterpret_cast<const uint16_t *>(raw), N, reinterpret_cast<uint16_t *>(w16), ldw,
+                       gw.lg_lanes, (unsigned)gw.col_blocks);
     return hipGetLastError();
 }
 

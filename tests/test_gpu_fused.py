@@ -425,6 +425,27 @@ def test_mul_mat_f16_forms(M, K, N, off):
     assert (np.abs(host(y) - ref) <= K * 2.0 ** -24 * _f16_terms_abs(w16, x)).all()
 
 
+@pytest.mark.parametrize("K", [5, 40, 1001, 1152])
+def test_mul_mat_f16_x_at_any_float(K):
+    # x rows at every 4-byte boundary (pointer and stride) give the bits of
+    # 16-byte aligned ones
+    M, N = 37, 24
+    say(f"F16 mul_mat x alignment K={K}")
+    rng = np.random.default_rng(57)
+    wd = dev(rng.standard_normal((N, K)).astype(np.float16).view(np.uint16))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    wsb = s2x.lib.s2x_mul_mat_f16_workspace_size(K, N, M)
+    ws, ref = empty((wsb,), torch.uint8), None
+    for off, ldx in ((0, K + -K % 4), (1, K + -K % 4), (2, K + 1), (3, K + 3), (0, K)):
+        flat = np.full(off + M * ldx, np.nan, np.float32)
+        flat[off:].reshape(M, ldx)[:, :K] = x
+        xd, y = dev(flat), empty((M, N), torch.float32)
+        s2x.call("s2x_mul_mat_f16_f32", ptr(wd), K, N, ctypes.c_void_p(xd.data_ptr() + 4 * off), ldx, M, ptr(y),
+                 ptr(ws), ctypes.c_size_t(wsb), stream())
+        ref = host(y) if ref is None else ref
+        assert_same(host(y), ref, f"off={off} ldx={ldx}")
+
+
 def test_mul_mat_f16_many_rows():
     # more rows than one wave each allows a launch (2^32 threads)
     M, K, N = (1 << 26) + 3, 8, 1
