@@ -10,6 +10,7 @@
 
 #include "s2x_internal.h"
 #include "s2x_kernels.h"
+#include "s2x_plan.h"
 
 namespace s2x {
 
@@ -271,19 +272,9 @@ int s2x_mul_mat_q8_0_f32(const void *w_raw, int64_t K_pad, int64_t N, const floa
     return e == hipSuccess ? S2X_OK : hip_fail(e, "gemm launch");
 }
 
-static MulMatWs mul_mat_f16_ws_layout(int64_t K, int64_t N, int64_t M) {
-    const int64_t K_pad = round_up_i(K, QK_);
-    MulMatWs L;
-    L.w_off = 0;
-    L.xq_off = (size_t)round_up_i(N * K_pad * 2, 256);
-    L.ds_off = L.xq_off;
-    L.total = L.xq_off + (size_t)round_up_i(M * K_pad * 2, 256);
-    return L;
-}
-
 size_t s2x_mul_mat_f16_workspace_size(int64_t K, int64_t N, int64_t M) {
     if (K <= 0 || N <= 0 || M < 0) return 0;
-    return mul_mat_f16_ws_layout(K, N, M).total;
+    return (size_t)f16_mul_mat_plan(K, N, M, false).total;
 }
 
 int s2x_mul_mat_f16_f32(const void *w_raw, int64_t K, int64_t N, const float *x, int64_t ldx,
@@ -296,27 +287,21 @@ int s2x_mul_mat_f16_f32(const void *w_raw, int64_t K, int64_t N, const float *x,
         return fail(S2X_ERR_UNSUPPORTED, "mul_mat_f16_f32: shape too large");
     if (!w_raw || !x || !y || !workspace)
         return fail(S2X_ERR_INVALID_ARG, "mul_mat_f16_f32: null pointer");
-    const MulMatWs L = mul_mat_f16_ws_layout(K, N, M);
-    if (ws_bytes < L.total)
-        return fail(S2X_ERR_WORKSPACE, "mul_mat_f16_f32: workspace %zu < %zu bytes", ws_bytes, L.total);
+    const F16MulMatPlan L = f16_mul_mat_plan(K, N, M, aligned(w_raw, 16));
+    if (ws_bytes < (size_t)L.total)
+        return fail(S2X_ERR_WORKSPACE, "mul_mat_f16_f32: workspace %zu < %zu bytes", ws_bytes, (size_t)L.total);
     if (!aligned(workspace, 256) || !aligned(w_raw, 2) || !aligned(x, 4) || !aligned(y, 4))
         return fail(S2X_ERR_INVALID_ARG, "mul_mat_f16_f32: misaligned pointer");
-    const int64_t K_pad = round_up_i(K, QK_);
+    // (refused before the conversion writes the workspace)
+    if (!f16_ld_ok(L.ldx16) || !f16_ld_ok(L.ldw)) return hip_fail(hipErrorInvalidValue, "gemm launch");
     uint8_t *ws = (uint8_t *)workspace;
     hipStream_t s = (hipStream_t)stream;
-    // The GEMM reads the raw weight rows in place where they are 16-byte
-    // aligned; X then has the whole workspace for rows of whole 128-byte
-    // lines, if those fit.
-    const bool w_direct = K % 8 == 0 && aligned(w_raw, 16);
-    const int64_t ld_line = round_up_i(K, 64);
-    const bool x_lines = w_direct && (size_t)(M * ld_line * 2) <= L.total;
-    const int64_t ldx16 = x_lines ? ld_line : K_pad, ldw = w_direct ? K : K_pad;
-    _Float16 *x16 = (_Float16 *)(ws + (x_lines ? 0 : L.xq_off));
-    _Float16 *w16 = w_direct ? (_Float16 *)const_cast<void *>(w_raw) : (_Float16 *)(ws + L.w_off);
-    hipError_t e = launch_f16_operands(x, K, M, ldx, x16, ldx16, w_direct ? nullptr : w_raw, N, w16, ldw, s);
+    _Float16 *x16 = (_Float16 *)(ws + L.x_off);
+    _Float16 *w16 = L.w_direct ? (_Float16 *)const_cast<void *>(w_raw) : (_Float16 *)ws;
+    hipError_t e = launch_f16_operands(x, K, M, ldx, x16, L.ldx16, L.w_direct ? nullptr : w_raw, N, w16, L.ldw, s);
     if (e != hipSuccess) return hip_fail(e, "convert launch");
     EpiParams p{EPI_NONE, nullptr, nullptr, 0, 0, 0};
-    e = launch_gemm_f16(w16, ldw, K, N, x16, ldx16, M, y, N, p, s);
+    e = launch_gemm_f16(w16, L.ldw, K, N, x16, L.ldx16, M, y, N, p, s);
     return e == hipSuccess ? S2X_OK : hip_fail(e, "gemm launch");
 }
 

@@ -63,6 +63,7 @@
 // 23,328, where the matrix pipe and the VALU bound the loop, 1 to 3 %.
 #include "s2x_device.h"
 #include "s2x_kernels.h"
+#include "s2x_plan.h"
 
 #include <type_traits>
 #include <utility>
@@ -1705,8 +1706,8 @@ hipError_t launch_gemm_f16(const _Float16 *w16, int64_t ldw, int64_t K, int64_t 
     if (M == 0 || N == 0) return hipSuccess;
     const int64_t K8 = (K + 7) / 8 * 8;
     if (!w16 || !x16 || !y || K <= 0 || ldw < K8 || ldx < K8 || ldw % 8 || ldx % 8 || M > (1 << 30) ||
-        N > (1 << 30) || ((uintptr_t)w16 & 15) || ((uintptr_t)x16 & 15) || 128 * ldw * 2 > 0x7fffffff ||
-        128 * ldx * 2 > 0x7fffffff || 128 * ldy * 4 > 0x7fffffff)
+        N > (1 << 30) || ((uintptr_t)w16 & 15) || ((uintptr_t)x16 & 15) || !f16_ld_ok(ldw) || !f16_ld_ok(ldx) ||
+        128 * ldy * 4 > 0x7fffffff)
         return hipErrorInvalidValue;
     switch (epi.kind) {
     case EPI_NONE: return run_f16_form<EPI_NONE>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);

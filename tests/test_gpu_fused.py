@@ -446,6 +446,23 @@ def test_mul_mat_f16_x_at_any_float(K):
         assert_same(host(y), ref, f"off={off} ldx={ldx}")
 
 
+@pytest.mark.parametrize("K", [8388544, 8388552, 8388576])
+def test_mul_mat_f16_longest_rows(K):
+    # the longest rows the GEMM's 31-bit offsets take; sums of -1, 0, 1 are
+    # exact in f32
+    M, N = 3, 2
+    say(f"F16 mul_mat K={K}")
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(59)
+    xd = torch.randint(-1, 2, (M, K), generator=g, device="cuda:0").float()
+    wd = torch.randint(-1, 2, (N, K), generator=g, device="cuda:0").to(torch.float16)
+    wsb = s2x.lib.s2x_mul_mat_f16_workspace_size(K, N, M)
+    ws, y = empty((wsb,), torch.uint8), empty((M, N), torch.float32)
+    s2x.call("s2x_mul_mat_f16_f32", ptr(wd), K, N, ptr(xd), K, M, ptr(y), ptr(ws), ctypes.c_size_t(wsb), stream())
+    ref = torch.stack([(xd * w.float()).double().sum(1) for w in wd], 1)
+    assert_same(host(y), ref.float().cpu().numpy(), f"K={K}")
+
+
 def test_mul_mat_f16_many_rows():
     # more rows than one wave each allows a launch (2^32 threads)
     M, K, N = (1 << 26) + 3, 8, 1

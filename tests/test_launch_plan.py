@@ -54,3 +54,28 @@ def test_f16_operand_grid_takes_rows_up_to_the_launch_limit(plan):
         rows = min(1 << 30, ((1 << 32) - 256) * 4 // k_pad)
         for ld in (k_pad, _up(K, 64)):
             assert _operand_grid(plan, rows, ld)[2] * 256 < 1 << 32, (K, ld, rows)
+
+
+def _f16_plan(plan, K, N, M, w_align16):
+    out = (ctypes.c_int64 * 5)()
+    plan.plan_f16_mul_mat(*(ctypes.c_int64(v) for v in (K, N, M)), int(w_align16), out)
+    return tuple(out)
+
+
+def test_f16_mul_mat_layouts_fit_the_workspace_and_the_gemm(plan):
+    # (K = 8,388,552 among them: its rows padded to 32 are within the GEMM's
+    # stride limit, rows of whole lines are not)
+    for K in (1, 7, 8, 24, 32, 40, 64, 72, 1001, 1076, 1152, 4304, 8388480, 8388488, 8388544, 8388552, 8388576):
+        k_pad = _up(K, 32)
+        assert plan.plan_f16_ld_ok(ctypes.c_int64(k_pad))
+        for N, M in ((1, 1), (1, 3), (2, 300), (300, 2), (1152, 729)):
+            for al in (0, 1):
+                direct, ldx, ldw, x_off, total = _f16_plan(plan, K, N, M, al)
+                assert total == _up(N * k_pad * 2, 256) + _up(M * k_pad * 2, 256)  # part of the interface
+                assert direct == (al and K % 8 == 0)
+                assert ldw == (K if direct else k_pad) and ldx >= K and ldx % 8 == 0
+                assert plan.plan_f16_ld_ok(ctypes.c_int64(ldx)), (K, N, M, al)
+                assert x_off % 256 == 0 and x_off + M * ldx * 2 <= total
+                assert direct or x_off >= N * ldw * 2  # the repacked rows lie in front
+    assert _f16_plan(plan, 4304, 1152, 2916, 1)[1] == 4352  # whole lines
+    assert not plan.plan_f16_ld_ok(ctypes.c_int64(8388608))
