@@ -279,18 +279,29 @@ __device__ __forceinline__ void epilogue(float (&acc)[TM][TN][16], float scale, 
         const bool vec = epi.h_ld % 8 == 0 && (reinterpret_cast<uintptr_t>(epi.h_out) & 15) == 0;  // uniform
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
+            const int rows = M - mw - a * 32;  // wave-uniform
+            auto gelu_rows = [&](auto whole) {
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+                for (int b = 0; b < 2; ++b)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    scr[(8 * (r >> 2) + 4 * lh + (r & 3)) * P + b * 32 + lr] =
-                        nw + b * 32 + lr < N ? f32_to_f16(gelu_tanh(fmaf(acc[a][b][r], scale, bias_v[b])))
-                                             : (_Float16)0.0f;
+                    for (int r = 0; r < 16; ++r) {
+                        const int r0 = 8 * (r >> 2) + (r & 3);  // rows r0 (lanes 0..31) and r0 + 4
+                        if (!decltype(whole)::value && r0 >= rows) continue;
+                        scr[(r0 + 4 * lh) * P + b * 32 + lr] =
+                            nw + b * 32 + lr < N ? f32_to_f16(gelu_tanh(fmaf(acc[a][b][r], scale, bias_v[b])))
+                                                 : (_Float16)0.0f;
+                    }
+            };
+            // (of a few rows only those: at M = 1 all 32 take 1.9 us longer)
+            if (rows >= 32)
+                gelu_rows(std::true_type{});
+            else
+                gelu_rows(std::false_type{});
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int id = lane + 64 * i, row = id >> 3, c = (id & 7) * 8;
                 const int m = mw + a * 32 + row, n = nw + c;
-                if (m >= M || n >= epi.h_kpad) continue;  // (h_kpad is a multiple of 32: whole chunks)
+                if (row >= rows || n >= epi.h_kpad) continue;  // (h_kpad is a multiple of 32: whole chunks)
                 _Float16 *dst = epi.h_out + (int64_t)m * epi.h_ld + n;
                 const v8h v = *reinterpret_cast<const v8h *>(scr + row * P + c);
                 if (vec) {

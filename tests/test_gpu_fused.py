@@ -506,3 +506,36 @@ def test_gelu_f16_epilogue(orc, weights, M):
     rq, rd = orc.quantize_q8_1(x[rows], K_pad)
     ref = orc.gelu(orc.mul_mat_q8_0_q8_1(raw, K_pad, N, rq, rd) + bias).astype(np.float16)
     assert_same(hg[rows, :N].view(np.uint16), ref.view(np.uint16), "GELU_F16 vs oracle")
+
+
+@pytest.mark.parametrize("M", [1, 5, 9, 31, 33, 150, 1100])
+@pytest.mark.parametrize("N", [72, 500])
+@pytest.mark.parametrize("off", [0, 1, 8])
+def test_gelu_f16_epilogue_ragged(orc, M, N, off):
+    # rows and columns past the tile's last ones are not written, at 16-byte
+    # stores (off: halves the output starts past alignment; 0, 8) and at
+    # 2-byte ones (1); M = 1100 fills whole 32-row halves
+    K, NP = 160, N + -N % 32
+    say(f"GELU->f16 epilogue M={M} N={N} off={off}")
+    rng = np.random.default_rng(55)
+    raw = synth.quantize_q8_0(rng.normal(0, 0.05, (N, K)).astype(np.float32), K)
+    bias = rng.standard_normal(N).astype(np.float32)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    qs, ds = _quant_gpu(x, K)
+    bd = dev(bias)
+    buf = torch.full((off + (M + 32) * NP,), 7.0, dtype=torch.float16, device="cuda:0")
+    w = _weight(raw, K, N)
+    try:
+        e = s2x.Epilogue()
+        e.kind, e.bias = s2x.EPI_GELU_F16, bd.data_ptr()
+        e.q_out, e.q_kpad = buf.data_ptr() + 2 * off, NP
+        s2x.call("s2x_mul_mat_q8_0_q8_1", w, ptr(qs), ptr(ds), M, None, 0, ctypes.byref(e), stream())
+        hg = host(buf)
+    finally:
+        s2x.lib.s2x_weight_destroy(w)
+    assert (hg[:off] == 7.0).all() and (hg[off + M * NP:] == 7.0).all()
+    got = hg[off:off + M * NP].reshape(M, NP)
+    assert not got[:, N:].view(np.uint16).any()
+    rq, rd = orc.quantize_q8_1(x, K)
+    ref = orc.gelu(orc.mul_mat_q8_0_q8_1(raw, K, N, rq, rd) + bias).astype(np.float16)
+    assert_same(got[:, :N].view(np.uint16), ref.view(np.uint16), f"GELU_F16 M={M} N={N} off={off}")
