@@ -1575,44 +1575,23 @@ static hipError_t run_gemv_epi(const WeightView &w, const int8_t *xq, const uint
         return hipErrorInvalidValue;  // (use_gemv admits no other epilogue)
 }
 
-// Stage configurations: 4-block stages in a ring of 2.  Wide: 128 x 128
-// tiles, two workgroups per CU, for GEMMs of enough tiles to fill the chip.
-// Small: the latency form, for GEMMs of fewer 128 x 128 tiles than two per
-// CU.  Each output's K order is the same in all, so the choice does not
-// change a bit (M = 729 in 128 x 128 tiles: out 19.8 us, fc2 58.7).
+// The tile forms (q8_form has the rule).  4-block stages; Wide in a ring of
+// two, the latency forms of up to four.
 #ifndef S2X_WIDE_TM
 #define S2X_WIDE_TM 1
 #endif
 using Wide = gemm::Cfg<4, 2, 128, false, S2X_WIDE_TM>;
-// The latency form's ring: four stages (three in flight) where its
-// workgroups fit one per CU, three stages (two per CU) otherwise.  The plain
-// / bias / residual epilogues (the out projection, fc2, the text tower's
-// QKV) run waves of 32 x 32 outputs, in the smallest tiles that still give
-// every workgroup a CU of its own (a workgroup's DMA, about 40 bytes per ns
-// from past the L2, is what a smaller tile shortens): one wave (Lone), two
-// (Narrow), else 64 x 64 tiles of four while all are resident, two per CU
-// (Square: 16 KB of quants a stage where 32 x 128 tiles take 20).  K = 4320,
-// N = 1152: M = 64 Lone 16.4 us, Narrow 17.0, Square 17.5; M = 320 Narrow
-// 18.1 to 18.6, Lone 18.4, Square 18.7; M = 729 Square 20.2, 32 x 128 20.5,
-// Narrow 25.3, Lone 33.4.  K = 1152: M = 320, N = 3456 Square 10.4, Narrow
-// 13.9, 32 x 128 14.3; M = 1458, N = 1152 Square 11.6, 32 x 128 15.6.  More
-// than two Square workgroups per CU: 64 x 128 tiles of waves with two
-// subtiles (M = 1800: 43.1 us, 46.0 before).  The same per-output K order in
-// all, without splitting K.
 using Small4 = gemm::Cfg<4, 4, 64, true>;
 using Small3 = gemm::Cfg<4, 3, 64, true>;
 using Lone = gemm::Cfg<4, 4, 32, true, 1, 1, 32>;
 using Narrow = gemm::Cfg<4, 4, 32, true, 1, 1, 64>;
 using Square = gemm::Cfg<4, 4, 64, true, 1, 1, 64>;
+using Rows32 = gemm::Cfg<4, 4, 32, true, 1, 1>;
 
 template <int E>
-static hipError_t run_small(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds,
+static hipError_t run_tiled(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds,
                             int64_t ld_ds, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
                             hipStream_t stream);
-
-static bool use_small(int64_t M, int64_t N) {
-    return ((M + 127) / 128) * ((N + 127) / 128) < 2 * 256;
-}
 
 hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xds, int64_t ld_ds,
                        int64_t M, float *y, int64_t ldy, const EpiParams &epi_in,
@@ -1633,8 +1612,7 @@ hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xd
         return hipErrorInvalidValue;
 #define S2X_RUN(E)                                                                     \
     (use_gemv(M, ldx, w, epi) ? run_gemv_epi<E>(w, xq, xds, ld_ds, M, y, ldy, epi, stream)  \
-     : !use_small(M, w.N) ? gemm::run<C, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream) \
-                          : run_small<E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream))
+                              : run_tiled<E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream))
     switch (epi.kind) {
     case EPI_NONE: return S2X_RUN(EPI_NONE);
     case EPI_BIAS: return S2X_RUN(EPI_BIAS);
@@ -1669,18 +1647,20 @@ hipError_t launch_gemm(const WeightView &w, const int8_t *xq, const uint32_t *xd
 }
 
 template <int E>
-static hipError_t run_small(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds,
+static hipError_t run_tiled(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds,
                             int64_t ld_ds, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
                             hipStream_t stream) {
     constexpr bool plain = E == EPI_NONE || E == EPI_BIAS || E == EPI_BIAS_GELU || E == EPI_BIAS_RESID ||
                            E == EPI_DUMP_I;
-    const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((w.N + bn - 1) / bn); };
+    const Q8Form form = q8_form(M, w.N, plain);
+    if (form == Q8Form::Wide) return gemm::run<Wide, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
     if constexpr (plain) {
-        if (tiles(32, 32) <= 256) return gemm::run<Lone, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
-        if (tiles(32, 64) <= 256) return gemm::run<Narrow, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
-        if (tiles(64, 64) <= 512) return gemm::run<Square, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        if (form == Q8Form::Lone) return gemm::run<Lone, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        if (form == Q8Form::Narrow) return gemm::run<Narrow, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        if (form == Q8Form::Square) return gemm::run<Square, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        if (form == Q8Form::Rows32) return gemm::run<Rows32, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
     } else {
-        if (tiles(64, 128) <= 256) return gemm::run<Small4, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
+        if (form == Q8Form::Small4) return gemm::run<Small4, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
     }
     return gemm::run<Small3, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
 }

@@ -61,4 +61,46 @@ inline F16MulMatPlan f16_mul_mat_plan(int64_t K, int64_t N, int64_t M, bool w_al
     return p;
 }
 
+// The tile form of a tiled int8 product (s2x_gemm.hip).  Each output's K order
+// is the same in all of them, so the choice does not change a bit.
+enum class Q8Form {
+    Wide,    // 128 x 128, the throughput form, two workgroups per CU
+    Lone,    // latency forms of 32 x 32 waves: 32 x 32, one wave
+    Narrow,  //   32 x 64, two waves
+    Square,  //   64 x 64, four waves, two workgroups per CU
+    Rows32,  //   32 x 128, four waves
+    Small4,  // latency forms of 32 x 64 waves: 64 x 128, four stages, one workgroup per CU
+    Small3   //   64 x 128, three stages, two workgroups per CU
+};
+// Wide for GEMMs of at least two 128 x 128 tiles per CU; below that the
+// latency form (M = 729 in 128 x 128 tiles: out 19.8 us, fc2 58.7).  The
+// epilogues that work on 32 x 64 blocks (plain false: GELU -> Q8_1 / F16, QKV)
+// have the 64 x 128 tiles, with four stages in the ring (three in flight)
+// where their workgroups fit one per CU and three stages (two per CU)
+// otherwise.  The plain / bias / residual ones (the out projection, fc2, the
+// text tower's QKV) run the smallest tiles that still give every workgroup a
+// CU of its own (a workgroup's DMA, about 40 bytes per ns from past the L2,
+// is what a smaller tile shortens), then Square while all of them are
+// resident: 16 KB of quants a stage where Rows32 takes 20.  Where Square is
+// past one workgroup per CU, a few CUs have two and the others wait for them:
+// Rows32 if that still is within one (K = 4320, N = 4304, M = 200: Rows32
+// 18.2 us, Square 23.8, Narrow 23.7, Lone 25.9; K = 1152 7.7, 9.4, 9.4, 8.7).
+// K = 4320, N = 1152: M = 64 Lone 16.4 us, Narrow 17.0, Square 17.5; M = 320
+// Narrow 18.1 to 18.6, Lone 18.4, Square 18.7; M = 729 Square 20.2, Rows32
+// 20.5, Narrow 25.3, Lone 33.4.  K = 1152: M = 320, N = 3456 Square 10.4,
+// Narrow 13.9, Rows32 14.3; M = 1458, N = 1152 Square 11.6, Rows32 15.6.  More
+// than two Square workgroups per CU: 64 x 128 tiles of waves with two
+// subtiles (M = 1800: 43.1 us).
+inline Q8Form q8_form(int64_t M, int64_t N, bool plain) {
+    const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    if (tiles(128, 128) >= 2 * 256) return Q8Form::Wide;
+    if (!plain) return tiles(64, 128) <= 256 ? Q8Form::Small4 : Q8Form::Small3;
+    if (tiles(32, 32) <= 256) return Q8Form::Lone;
+    if (tiles(32, 64) <= 256) return Q8Form::Narrow;
+    if (tiles(64, 64) <= 256) return Q8Form::Square;
+    if (tiles(32, 128) <= 256) return Q8Form::Rows32;
+    if (tiles(64, 64) <= 512) return Q8Form::Square;
+    return Q8Form::Small3;
+}
+
 }  // namespace s2x

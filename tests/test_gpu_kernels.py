@@ -8,6 +8,7 @@ import torch
 
 import s2x
 from s2x import synth
+from gemm_forms import LATENCY_SHAPES
 from gpu_util import assert_same, cos, dev, empty, host, ptr, say, stream, zeros
 
 pytestmark = pytest.mark.gpu
@@ -284,6 +285,45 @@ def test_gemm_latency_forms(orc, M, N, KB):
         y = empty((M, N), torch.float32)
         s2x.call("s2x_mul_mat_q8_0_q8_1", w, ptr(qs), ptr(ds), M, ptr(y), N, None, stream())
         assert_same(host(y)[rows], ref, f"gemm KB={KB} M={M} N={N}")
+    finally:
+        s2x.lib.s2x_weight_destroy(w)
+
+
+# Every tile form of the latency GEMM (test_launch_plan.py checks that the
+# shapes take them) at ragged edges, with 1 to 5 stages of 4 blocks: shorter
+# than a stage, than the ring, and long enough that a released slot is
+# refilled with live data (17 blocks and more in a ring of four stages, 13
+# in one of three) before a last stage of 1, 2, 3 and 4 blocks.  Sums and
+# GELU -> Q8_1 are the oracle's bits.
+@pytest.mark.parametrize("KB", [1, 2, 3, 4, 5, 8, 13, 17, 18, 19, 20])
+@pytest.mark.parametrize("form,M,N,plain", LATENCY_SHAPES)
+def test_gemm_tile_forms(orc, form, M, N, plain, KB):
+    K = 32 * KB
+    say(f"gemm form {form}: KB={KB} M={M} N={N} plain={plain}")
+    rng = np.random.default_rng(95 + KB)
+    raw = synth.quantize_q8_0(rng.normal(0, 0.02, (N, K)).astype(np.float32), K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    qs, ds = _quant_gpu(x, K)
+    rows = np.arange(M) if M < 80 else np.unique(np.concatenate([rng.choice(M, 24, replace=False), np.arange(M - 40, M)]))
+    rq, rd = orc.quantize_q8_1(x[rows], K)
+    ref = orc.mul_mat_q8_0_q8_1(raw, K, N, rq, rd)
+    w = _weight(raw, K, N)
+    try:
+        if plain:
+            y = empty((M, N), torch.float32)
+            s2x.call("s2x_mul_mat_q8_0_q8_1", w, ptr(qs), ptr(ds), M, ptr(y), N, None, stream())
+            assert_same(host(y)[rows], ref, f"{form} KB={KB}")
+            return
+        NP, bd = N + -N % 32, dev(bias)
+        q, d = empty((M, NP), torch.int8), empty((M, NP // 32), torch.int32)
+        e = s2x.Epilogue()
+        e.kind, e.bias = s2x.EPI_GELU_Q81, bd.data_ptr()
+        e.q_out, e.q_ds, e.q_kpad = q.data_ptr(), d.data_ptr(), NP
+        s2x.call("s2x_mul_mat_q8_0_q8_1", w, ptr(qs), ptr(ds), M, None, 0, ctypes.byref(e), stream())
+        gq, gd = orc.quantize_q8_1(orc.gelu_mode(orc.GELU_EXACT, ref + bias), NP)
+        assert_same(host(q)[rows], gq, f"{form} KB={KB} quants")
+        assert_same(host(d)[rows], gd.view(np.int32)[..., 0], f"{form} KB={KB} ds")
     finally:
         s2x.lib.s2x_weight_destroy(w)
 

@@ -8,6 +8,8 @@ import subprocess
 import numpy as np
 import pytest
 
+from gemm_forms import LATENCY_SHAPES
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "hbd-siglip2.cpp_amd", "csrc")
 
@@ -79,3 +81,30 @@ def test_f16_mul_mat_layouts_fit_the_workspace_and_the_gemm(plan):
                 assert direct or x_off >= N * ldw * 2  # the repacked rows lie in front
     assert _f16_plan(plan, 4304, 1152, 2916, 1)[1] == 4352  # whole lines
     assert not plan.plan_f16_ld_ok(ctypes.c_int64(8388608))
+
+
+Q8_FORMS = ["Wide", "Lone", "Narrow", "Square", "Rows32", "Small4", "Small3"]
+
+
+def _q8_form(plan, M, N, plain=True):
+    return Q8_FORMS[plan.plan_q8_form(ctypes.c_int64(M), ctypes.c_int64(N), int(plain))]
+
+
+@pytest.mark.parametrize("form,M,N,plain", LATENCY_SHAPES)
+def test_latency_shapes_take_their_form(plan, form, M, N, plain):
+    # the shapes of the GPU tests of each tile form
+    assert _q8_form(plan, M, N, plain) == form
+
+
+def test_q8_form_fills_the_cus_once(plan):
+    # a plain product within one workgroup per CU of some form is not given
+    # to one that puts two on a few CUs (M = 200, N = 4,304 took 23.8 us that
+    # way, 18.2 in 32 x 128 tiles)
+    dims = {"Lone": (32, 32), "Narrow": (32, 64), "Square": (64, 64), "Rows32": (32, 128)}
+    for M in range(9, 1500, 13):
+        for N in (64, 256, 768, 1152, 2304, 3456, 4304):
+            tiles = {f: -(-M // bm) * -(-N // bn) for f, (bm, bn) in dims.items()}
+            got = _q8_form(plan, M, N)
+            if min(tiles.values()) <= 256:
+                assert tiles[got] <= 256, (M, N, got, tiles)
+            assert _q8_form(plan, M, N, False) in ("Wide", "Small4", "Small3")
