@@ -1652,7 +1652,8 @@ static hipError_t run_tiled(const WeightView &w, const int8_t *xq, int64_t ldx, 
                             hipStream_t stream) {
     constexpr bool plain = E == EPI_NONE || E == EPI_BIAS || E == EPI_BIAS_GELU || E == EPI_BIAS_RESID ||
                            E == EPI_DUMP_I;
-    const Q8Form form = q8_form(M, w.N, plain);
+    const int64_t KB = w.K_pad / QK;
+    const Q8Form form = q8_form(M, w.N, plain, epi.kb_split > 0 ? (KB + epi.kb_split - 1) / epi.kb_split : 1);
     if (form == Q8Form::Wide) return gemm::run<Wide, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
     if constexpr (plain) {
         if (form == Q8Form::Lone) return gemm::run<Lone, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);

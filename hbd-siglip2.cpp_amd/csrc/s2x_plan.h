@@ -91,15 +91,20 @@ enum class Q8Form {
 // Narrow 13.9, Rows32 14.3; M = 1458, N = 1152 Square 11.6, Rows32 15.6.  More
 // than two Square workgroups per CU: 64 x 128 tiles of waves with two
 // subtiles (M = 1800: 43.1 us).
-inline Q8Form q8_form(int64_t M, int64_t N, bool plain) {
-    const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    if (tiles(128, 128) >= 2 * 256) return Q8Form::Wide;
+// A K split has n_split workgroups per tile, which count for what fits one per
+// CU; Square and Wide end by the tiles of one range.  Counting those alone
+// everywhere gave Narrow to K = 4320, N = 256, M = 1458 in 2 ranges: 17.7 us,
+// Square 14.1.
+inline Q8Form q8_form(int64_t M, int64_t N, bool plain, int64_t n_split = 1) {
+    const auto grid = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const auto tiles = [&](int64_t bm, int64_t bn) { return grid(bm, bn) * n_split; };
+    if (grid(128, 128) >= 2 * 256) return Q8Form::Wide;
     if (!plain) return tiles(64, 128) <= 256 ? Q8Form::Small4 : Q8Form::Small3;
     if (tiles(32, 32) <= 256) return Q8Form::Lone;
     if (tiles(32, 64) <= 256) return Q8Form::Narrow;
     if (tiles(64, 64) <= 256) return Q8Form::Square;
     if (tiles(32, 128) <= 256) return Q8Form::Rows32;
-    if (tiles(64, 64) <= 512) return Q8Form::Square;
+    if (grid(64, 64) <= 512) return Q8Form::Square;
     return Q8Form::Small3;
 }
 

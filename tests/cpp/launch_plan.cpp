@@ -11,5 +11,7 @@ void plan_f16_mul_mat(int64_t K, int64_t N, int64_t M, int w_align16, int64_t *o
     out[0] = p.w_direct, out[1] = p.ldx16, out[2] = p.ldw, out[3] = p.x_off, out[4] = p.total;
 }
 int plan_f16_ld_ok(int64_t ld) { return s2x::f16_ld_ok(ld); }
-int plan_q8_form(int64_t M, int64_t N, int plain) { return (int)s2x::q8_form(M, N, plain != 0); }
+int plan_q8_form(int64_t M, int64_t N, int plain, int64_t n_split) {
+    return (int)s2x::q8_form(M, N, plain != 0, n_split);
+}
 }

@@ -86,8 +86,8 @@ def test_f16_mul_mat_layouts_fit_the_workspace_and_the_gemm(plan):
 Q8_FORMS = ["Wide", "Lone", "Narrow", "Square", "Rows32", "Small4", "Small3"]
 
 
-def _q8_form(plan, M, N, plain=True):
-    return Q8_FORMS[plan.plan_q8_form(ctypes.c_int64(M), ctypes.c_int64(N), int(plain))]
+def _q8_form(plan, M, N, plain=True, n_split=1):
+    return Q8_FORMS[plan.plan_q8_form(ctypes.c_int64(M), ctypes.c_int64(N), int(plain), ctypes.c_int64(n_split))]
 
 
 @pytest.mark.parametrize("form,M,N,plain", LATENCY_SHAPES)
@@ -96,15 +96,16 @@ def test_latency_shapes_take_their_form(plan, form, M, N, plain):
     assert _q8_form(plan, M, N, plain) == form
 
 
-def test_q8_form_fills_the_cus_once(plan):
+@pytest.mark.parametrize("n_split", [1, 2, 4, 16])
+def test_q8_form_fills_the_cus_once(plan, n_split):
     # a plain product within one workgroup per CU of some form is not given
     # to one that puts two on a few CUs (M = 200, N = 4,304 took 23.8 us that
-    # way, 18.2 in 32 x 128 tiles)
+    # way, 18.2 in 32 x 128 tiles); a K split has n_split workgroups per tile
     dims = {"Lone": (32, 32), "Narrow": (32, 64), "Square": (64, 64), "Rows32": (32, 128)}
     for M in range(9, 1500, 13):
         for N in (64, 256, 768, 1152, 2304, 3456, 4304):
-            tiles = {f: -(-M // bm) * -(-N // bn) for f, (bm, bn) in dims.items()}
-            got = _q8_form(plan, M, N)
+            tiles = {f: -(-M // bm) * -(-N // bn) * n_split for f, (bm, bn) in dims.items()}
+            got = _q8_form(plan, M, N, True, n_split)
             if min(tiles.values()) <= 256:
                 assert tiles[got] <= 256, (M, N, got, tiles)
             assert _q8_form(plan, M, N, False) in ("Wide", "Small4", "Small3")
