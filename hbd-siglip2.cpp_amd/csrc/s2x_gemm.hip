@@ -111,7 +111,7 @@ struct Cfg {
     static constexpr int WG_PER_CU = 2 * LDS_BYTES <= 163840 ? 2 : 1;
     static constexpr int WPE = LAT ? 2 : WG_PER_CU * NWAVE / 4;  // waves per SIMD
     // DMA instructions per stage: QPX X-quant and QPW W-quant per wave (each
-    // 8 rows of the stage's KS blocks: BM / 8 and 16 per stage); the scales, 16
+    // 8 rows of the stage's KS blocks: BM / 8 and BN / 8 per stage); the scales, 16
     // bytes per lane (a row's 4 consecutive ds words, or 8 W scales of one
     // block), by the first NSX + 1 waves: waves 0 .. NSX - 1 the X scales
     // of 64 rows each, wave NSX the W scales.  The issue cost of these
@@ -755,14 +755,13 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // 0..3, lanes 32..63 (slots 4..7) zero: the products sum to -c0
     const v2i cA = {lh ? 0 : (int)0xC45FB000u, lh ? 0 : 0xAA0C};
     const v2i cB = {lh ? 0 : 0x20003C00, lh ? 0 : 0x0800};
-    // hook(): called once the block's last block dot is issued (where the
-    // throughput form reads the next block's fragments)
+    // (The throughput form's, and the block-dot dump's in either form; the
+    // latency form's blocks are the slots below.)  hook(): called once the
+    // block's last block dot is issued (where the throughput form reads the
+    // next block's fragments).
     auto compute = [&](const Frag<TM, TN> &f, int kb, auto &&hook) {
         const v16f zf = {};
         const v16i zi = {};
-        // c0's bits in every element (the latency form's splat; the
-        // throughput form names the inline constant itself, below)
-        const v16i magic = 0x3E22F983;
         if constexpr (EPI == EPI_DUMP_I) {
 #pragma unroll
             for (int k = 0; k < NSUB; ++k) {
@@ -784,23 +783,19 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             for (int k = 0; k < NSUB; ++k) {
                 const int a = k / TN, b = k % TN;
                 v16i D;
-                if constexpr (!C::LAT) {
-                    // The accumulator operand as the inline constant 1/2pi
-                    // (0x3E22F983) in the instruction: LLVM folds the splat
-                    // only where one MFMA uses it, and otherwise keeps it in
-                    // 16 VGPRs that every block dot reads -- at <= 128 VGPRs
-                    // for 4 waves per SIMD.  Written this way the K loop
-                    // takes ~100 VGPRs.  The one reader of D is the
-                    // conversion MFMA right below, with D exactly as its
-                    // accumulator operand: the dependency the compiler
-                    // itself schedules back to back with no wait states
-                    // (an MFMA whose srcC exactly overlaps the previous
-                    // MFMA's result); no VALU instruction reads D.
-                    asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0.15915494"
-                                 : "=&v"(D) : "v"(f.a[a]), "v"(f.b[b]));
-                } else {
-                    D = __builtin_amdgcn_mfma_i32_32x32x32_i8(f.a[a], f.b[b], magic, 0, 0, 0);
-                }
+                // The accumulator operand as the inline constant 1/2pi
+                // (0x3E22F983) in the instruction: LLVM folds the splat
+                // only where one MFMA uses it, and otherwise keeps it in
+                // 16 VGPRs that every block dot reads -- at <= 128 VGPRs
+                // for 4 waves per SIMD.  Written this way the K loop
+                // takes ~100 VGPRs.  The one reader of D is the
+                // conversion MFMA right below, with D exactly as its
+                // accumulator operand: the dependency the compiler
+                // itself schedules back to back with no wait states
+                // (an MFMA whose srcC exactly overlaps the previous
+                // MFMA's result); no VALU instruction reads D.
+                asm volatile("v_mfma_i32_32x32x32_i8 %0, %1, %2, 0.15915494"
+                             : "=&v"(D) : "v"(f.a[a]), "v"(f.b[b]));
                 if (k == NSUB - 1) hook();
                 const v16f I = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, cA),
                                                                     __builtin_bit_cast(v4h, cB),
@@ -811,8 +806,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
                 for (int r = 0; r < 16; ++r) acc[a][b][r] = fmaf(I[r], S[r], acc[a][b][r]);
             }
         }
-        // throughput form: one scheduling region per block, nothing moves
-        // across blocks
+        // one scheduling region per block, nothing moves across blocks
         if constexpr (!C::LAT) __builtin_amdgcn_sched_barrier(0);
     };
 
@@ -1016,7 +1010,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     }
     issue(0, role, All{}, std::true_type{});
     arrive();  // the first stage visible
-    if constexpr (C::LAT) issue(1, role, All{}, std::false_type{});
+    if constexpr (C::LAT) issue(1, role, All{}, std::false_type{});  // (here and below: the block-dot dump)
     // stage g computed while stage g + 1 loads; each block's fragments are
     // read right before its MFMAs (the other waves of the SIMD cover the
     // LDS latency)
@@ -1047,9 +1041,8 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
             });
         }
         arrive();
-        // the latency form's MFMAs may sink below the barrier (its stage is
-        // one scheduling region): its next DMA goes out after the barrier,
-        // a whole stage before the wait for it
+        // the latency form's stage is one scheduling region here: its next
+        // DMA goes out after the barrier, a whole stage before the wait for it
         if constexpr (C::LAT) issue(g + 2, role, All{}, std::false_type{});
     }
     {
@@ -1650,6 +1643,8 @@ template <int E>
 static hipError_t run_tiled(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_t *xds,
                             int64_t ld_ds, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
                             hipStream_t stream) {
+    // (the block-dot dump too: K = 4320, N = 1152, M = 64 12.5 us, in the 64 x
+    // 128 forms alone 15.9)
     constexpr bool plain = E == EPI_NONE || E == EPI_BIAS || E == EPI_BIAS_GELU || E == EPI_BIAS_RESID ||
                            E == EPI_DUMP_I;
     const int64_t KB = w.K_pad / QK;
