@@ -1,14 +1,15 @@
-"""The throughput GEMM writes its int8 block dot as inline assembly
-(`v_mfma_i32_32x32x32_i8 ..., 0.15915494`: the accumulator operand as the
-inline constant 1/2pi), which the compiler's hazard recognizer does not
-see.  That is sound because the only reader of each block dot's result is
+"""The int8 GEMM, its throughput form and the K loop of its latency forms,
+writes the int8 block dot as inline assembly (`v_mfma_i32_32x32x32_i8 ...,
+0.15915494`: the accumulator operand as the inline constant 1/2pi), which the
+compiler's hazard recognizer does not see.  That is sound because the only reader of each block dot's result is
 the conversion MFMA that takes it, register for register, as its
 accumulator operand -- a dependency that needs no wait states (the compiler
 itself issues two such builtins back to back).  This test compiles
 s2x_gemm.hip to gfx950 assembly and checks, for every inline block dot,
 that the first later instruction touching any of its result registers is
-that conversion MFMA with exactly those registers as its accumulator; and,
-as the reference for "no wait states", that the compiler issues the
+that conversion MFMA with exactly those registers as its accumulator, that
+every kernel of every tile form has such dots, and that none of their operands
+is written by the VALU in the two instructions before; and, as the reference for "no wait states", that the compiler issues the
 builtin pair back to back."""
 import os
 import re
@@ -24,6 +25,12 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-I", os.path.join(ROOT, "include"), "-I", CSRC,
          "-x", "hip", "-mllvm", "-amdgpu-mfma-vgpr-form", "--cuda-device-only", "-S"]
+
+# tile forms (csrc/s2x_plan.h, Q8Form): KS, NS, BM, LAT, TM, TN, BN
+FORMS = {"Wide": (4, 2, 128, 0, 1, 2, 128), "Small3": (4, 3, 64, 1, 1, 2, 128), "Small4": (4, 4, 64, 1, 1, 2, 128),
+         "Lone": (4, 4, 32, 1, 1, 1, 32), "Narrow": (4, 4, 32, 1, 1, 1, 64), "Square": (4, 4, 64, 1, 1, 1, 64),
+         "Rows32": (4, 4, 32, 1, 1, 1, 128)}
+EPI_DUMP_I = 4  # csrc/s2x_kernels.h
 
 pytestmark = pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which("hipcc")),
                                 reason="hipcc is not installed")
@@ -52,6 +59,36 @@ def _instructions(asm):
         yield t
 
 
+def _kernels(asm):
+    """{mangled name: its instructions} of the int8 GEMM's kernels."""
+    out, cur = {}, None
+    for line in asm.splitlines():
+        m = re.match(r"(\w+):", line)
+        if m and m[1].startswith("_Z"):
+            cur = m[1]
+        elif line.startswith(".Lfunc_end"):
+            cur = None
+        elif cur and "6k_gemmI" in cur:
+            out.setdefault(cur, []).extend(_instructions(line))
+    return out
+
+
+def _form_of(kernel):
+    """Cfg's arguments (KS, NS, BM, LAT, TM, TN, BN) of a kernel's name, and its epilogue."""
+    m = re.search(r"3CfgILi(\d+)ELi(\d+)ELi(\d+)ELb(\d)ELi(\d+)ELi(\d+)ELi(\d+)EEELi(\d+)E", kernel)
+    assert m, kernel
+    return tuple(int(v) for v in m.groups()[:7]), int(m[8])
+
+
+def _valu_feeds(instrs, i):
+    """True if a VALU instruction just before the dot i (two wait states) writes
+    one of its operands."""
+    ops = _operands(instrs[i])
+    src = _regs(ops[1]) | _regs(ops[2])
+    return any(t.startswith("v_") and not t.startswith("v_mfma") and _regs(_operands(t)[0]) & src
+               for t in instrs[max(0, i - 2):i])
+
+
 def _first_toucher_ok(instrs, i, dst):
     """True if the first instruction after i that names a register of dst
     is a v_mfma_f32_32x32x8_f16 whose accumulator operand is exactly dst."""
@@ -71,12 +108,25 @@ def test_inline_block_dots_feed_only_their_conversion(tmp_path):
     r = subprocess.run([HIPCC, *FLAGS, os.path.join(CSRC, "s2x_gemm.hip"), "-o", str(out)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
-    instrs = list(_instructions(out.read_text()))
-    dots = [i for i, t in enumerate(instrs)
-            if t.startswith("v_mfma_i32_32x32x32_i8") and "0.15915494" in t]
-    assert dots, "no inline block dots in the throughput GEMM"
-    bad = [instrs[i] for i in dots if not _first_toucher_ok(instrs, i, _regs(_operands(instrs[i])[0]))]
-    assert not bad, f"{len(bad)} of {len(dots)} block dots have another first reader, e.g. {bad[0]}"
+    asm = out.read_text()
+    kernels = _kernels(asm)
+    forms = set()
+    for name, instrs in kernels.items():
+        cfg, epi = _form_of(name)
+        dots = [i for i, t in enumerate(instrs)
+                if t.startswith("v_mfma_i32_32x32x32_i8") and "0.15915494" in t]
+        if epi == EPI_DUMP_I:
+            assert not dots, name
+            continue
+        assert dots, f"no inline block dots in {name}"
+        forms.add(cfg)
+        bad = [instrs[i] for i in dots if not _first_toucher_ok(instrs, i, _regs(_operands(instrs[i])[0]))]
+        assert not bad, f"{len(bad)} of {len(dots)} block dots have another first reader, e.g. {bad[0]}"
+        fed = [instrs[i - 2:i + 1] for i in dots if _valu_feeds(instrs, i)]
+        assert not fed, f"{name}: operands written right before, e.g. {fed[0]}"
+    assert forms == set(FORMS.values()), forms
+    # none elsewhere
+    assert asm.count("0.15915494") == sum("0.15915494" in t for i in kernels.values() for t in i)
 
 
 @pytest.mark.timeout(300)
@@ -124,3 +174,5 @@ def test_the_scan_rejects_other_first_readers():
     assert not _first_toucher_ok([dot, copy, conv_ok], 0, dst)
     assert not _first_toucher_ok([dot, conv_part], 0, dst)
     assert not _first_toucher_ok([dot, other], 0, dst)
+    assert _valu_feeds(["v_mov_b32_e32 v21, v5", other, dot], 2)
+    assert not _valu_feeds(["v_mov_b32_e32 v21, v5", other, other, dot], 3)
