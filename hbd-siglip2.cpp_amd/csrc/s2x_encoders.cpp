@@ -368,8 +368,8 @@ struct Tower {
     }
 
     // Row stride of fc2's Q8_1 input: whole cache lines for the tiled GEMMs;
-    // the few-row form (at most 8 rows) takes rows back to back
-    int64_t ld_q2(int64_t M) const { return M <= 8 ? F_pad : gemm_ld_q(F_pad); }
+    // the few-rows form takes rows back to back
+    int64_t ld_q2(int64_t M) const { return M <= GEMM_FEW_ROWS ? F_pad : gemm_ld_q(F_pad); }
 
     // The MLP of a block or of the MAP head on M rows whose LN2 + Q8_1 is in
     // qs / ds: fc1 (+bias, GELU, and Q8_1 -- or f16 for an F16 ffn_down --

@@ -1375,7 +1375,6 @@ hipError_t launch_gemm_split_k(const WeightView &w, const int8_t *xq, const uint
 // residual epilogues: the head's N = 1,152 GEMMs in 144 workgroups), or 32
 // where the epilogue quantizes 32-column blocks (GELU -> Q8_1).
 // ---------------------------------------------------------------------------
-constexpr int GV_MAX_M = 8;
 constexpr int GV_NT = 256;
 constexpr int GV_IT = 8;    // (column, block) pairs per thread: CW KB <= 2,048
 constexpr int GV_XIT = 12;  // 16-byte X chunks per thread: M K_pad <= 49,152
@@ -1536,13 +1535,13 @@ static hipError_t run_gemv(const WeightView &w, const int8_t *xq, const uint32_t
     return hipGetLastError();
 }
 
-// The GEMV form takes M <= 8 rows with a plain, bias, GELU, residual (not
+// The GEMV form takes M <= GEMM_FEW_ROWS rows with a plain, bias, GELU, residual (not
 // the position rows) or GELU -> Q8_1 epilogue and no K split, where its
 // per-thread unrolls and LDS hold the sizes.
 template <int CW>
 static bool gv_fits(int64_t M, const WeightView &w) {
     const int64_t KB = w.K_pad / QK;
-    return M <= GV_MAX_M && CW * KB <= GV_IT * GV_NT && M * KB <= GV_IT * GV_NT &&
+    return M <= GEMM_FEW_ROWS && CW * KB <= GV_IT * GV_NT && M * KB <= GV_IT * GV_NT &&
            M * (w.K_pad / 16) <= GV_XIT * GV_NT && gv_lds_bytes<CW>(M, w.K_pad) <= GV_LDS_MAX;
 }
 static bool use_gemv(int64_t M, int64_t ldx, const WeightView &w, const EpiParams &epi) {

@@ -34,6 +34,10 @@ inline int64_t gemm_ld_q(int64_t K_pad) {
     return K_pad > (1 << 23) ? K_pad : (K_pad + 127) / 128 * 128;  // (a tile's rows stay within 31 bits)
 }
 
+// Most rows of the GEMM's few-rows form, which takes X rows back to back
+// (K_pad bytes apart).
+constexpr int64_t GEMM_FEW_ROWS = 8;
+
 // Column tile of the GEMM; the transposed weight scales are padded to it.
 constexpr int64_t GEMM_BN = 128;
 inline int64_t gemm_ld_dw(int64_t N) { return (N + GEMM_BN - 1) / GEMM_BN * GEMM_BN; }
