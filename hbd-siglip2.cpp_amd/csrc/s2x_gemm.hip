@@ -1660,14 +1660,7 @@ static hipError_t run_tiled(const WeightView &w, const int8_t *xq, int64_t ldx, 
     return gemm::run<Small3, E>(w, xq, ldx, xds, ld_ds, M, y, ldy, epi, stream);
 }
 
-// The form of an F16 product, by tiles per round of the 256 CUs (every form
-// gives the same bits).  Small: 64 x 64 tiles, two workgroups a CU, while all
-// of them are resident at once (M = 729, K = 4320, N = 1152: 18 us against
-// 33 in 128 x 128 tiles; at 648 tiles, M = 729, K = 1152, N = 3456: 14.6
-// against 12.4).  Above that 128 x 128 tiles, or 256 x 128 where that takes
-// fewer rounds by more than the 1.6 x that a round of them is longer: M =
-// 3645, K = 4320, N = 1152 (2 rounds or 1) 63 against 51 us, M = 8640 (3 or
-// 2) 103 against 107, M = 23,328 (7 or 4) 301 against 257.
+// The tile forms of the F16 GEMM (f16_form has the rule)
 using SmallH = gemm::CfgH<1, 1, 2, 2, 4>;
 using MidH = gemm::CfgH<1, 2, 4, 2, 4>;
 using WideH = gemm::CfgH<2, 2, 4, 2, 3>;
@@ -1676,14 +1669,11 @@ template <int E>
 static hipError_t run_f16_form(const _Float16 *w16, int64_t ldw, int64_t K, int64_t N, const _Float16 *x16,
                                int64_t ldx, int64_t M, float *y, int64_t ldy, const EpiParams &epi,
                                hipStream_t stream) {
-    const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    const auto rounds = [&](int64_t t) { return (t + 255) / 256; };
-    if (tiles(SmallH::BM, SmallH::BN) <= 512)
-        return gemm::run_f16<SmallH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
-    if (8 * rounds(tiles(WideH::BM, WideH::BN)) < 5 * rounds(tiles(MidH::BM, MidH::BN)) &&
-        WideH::BM * ldx * 2 <= 0x7fffffff)
-        return gemm::run_f16<WideH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
-    return gemm::run_f16<MidH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
+    switch (f16_form(M, N, ldx)) {
+    case F16Form::Small: return gemm::run_f16<SmallH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
+    case F16Form::Wide: return gemm::run_f16<WideH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
+    default: return gemm::run_f16<MidH, E>(w16, ldw, K, N, x16, ldx, M, y, ldy, epi, stream);
+    }
 }
 
 hipError_t launch_gemm_f16(const _Float16 *w16, int64_t ldw, int64_t K, int64_t N, const _Float16 *x16,

@@ -61,6 +61,24 @@ inline F16MulMatPlan f16_mul_mat_plan(int64_t K, int64_t N, int64_t M, bool w_al
     return p;
 }
 
+// The tile form of an F16 product, by tiles per round of the 256 CUs (every
+// form gives the same bits).  Small: 64 x 64 tiles, two workgroups a CU, while
+// all of them are resident at once (M = 729, K = 4320, N = 1152: 18 us against
+// 33 in 128 x 128 tiles; at 648 tiles, M = 729, K = 1152, N = 3456: 14.6
+// against 12.4).  Above that 128 x 128 tiles, or 256 x 128 where that takes
+// fewer rounds by more than the 1.6 x that a round of them is longer (and the
+// taller tile's rows lie within 31 bits): M = 3645, K = 4320, N = 1152 (2
+// rounds or 1) 63 against 51 us, M = 8640 (3 or 2) 103 against 107, M =
+// 23,328 (7 or 4) 301 against 257.
+enum class F16Form { Small, Mid, Wide };
+inline F16Form f16_form(int64_t M, int64_t N, int64_t ldx) {
+    const auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const auto rounds = [&](int64_t t) { return (t + 255) / 256; };
+    if (tiles(64, 64) <= 512) return F16Form::Small;
+    if (8 * rounds(tiles(256, 128)) < 5 * rounds(tiles(128, 128)) && 256 * ldx * 2 <= 0x7fffffff) return F16Form::Wide;
+    return F16Form::Mid;
+}
+
 // The tile form of a tiled int8 product (s2x_gemm.hip).  Each output's K order
 // is the same in all of them, so the choice does not change a bit.
 enum class Q8Form {

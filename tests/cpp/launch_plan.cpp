@@ -14,4 +14,5 @@ int plan_f16_ld_ok(int64_t ld) { return s2x::f16_ld_ok(ld); }
 int plan_q8_form(int64_t M, int64_t N, int plain, int64_t n_split) {
     return (int)s2x::q8_form(M, N, plain != 0, n_split);
 }
+int plan_f16_form(int64_t M, int64_t N, int64_t ldx) { return (int)s2x::f16_form(M, N, ldx); }
 }

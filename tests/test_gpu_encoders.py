@@ -11,6 +11,7 @@ import torch
 import pyoracle
 import s2x
 from s2x import synth
+from gemm_forms import F16_TOWER_ROWS
 from gpu_util import cos, dev, empty, host, ptr, say
 
 pytestmark = pytest.mark.gpu
@@ -439,6 +440,31 @@ def test_so400m_text_5x64_vs_oracle(orc):
             assert c >= 0.9999
     finally:
         t.close()
+
+
+def test_f16_ffn_down_forms_agree(orc):
+    # fc2 of an F16 file with its bias and residual in the three tile forms of
+    # the F16 GEMM (1, 4 and 32 images): the same bits, near the oracle
+    cfg = synth.VisionConfig(n_layer=1)
+    assert (cfg.hidden, cfg.inter) == (1152, 4304)
+    hm = synth.vision_model(cfg, seed=27, down_f16=True)
+    v = Vision(hm)
+    try:
+        px = synth.pixels(4, 729, seed=28)
+        images = {f: rows // 729 for f, rows in F16_TOWER_ROWS.items()}
+        say(f"F16 ffn_down forms: {images}")
+        alone = np.concatenate([v.batch(px[i * 729:(i + 1) * 729], images["Small"], 27, 27, s2x.POOL_PROBE)
+                                for i in range(4)])
+        mid = v.batch(px, images["Mid"], 27, 27, s2x.POOL_PROBE)
+        wide = v.batch(np.tile(px, (8, 1)), images["Wide"], 27, 27, s2x.POOL_PROBE)
+    finally:
+        v.close()
+    assert np.array_equal(mid, alone)
+    assert np.array_equal(wide, np.tile(alone, (8, 1)))
+    ref = orc.vision_encode(orc.vision_model(hm), px[:729], 27, 27, pooling=s2x.POOL_PROBE)
+    c = cos(alone[0], ref)
+    say(f"  cosine vs oracle {c:.7f}")
+    assert c >= 0.9999
 
 
 def test_small_towers_f16_ffn_down(orc, tmp_path):

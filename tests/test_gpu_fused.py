@@ -13,6 +13,7 @@ import torch
 
 import s2x
 from s2x import synth
+from gemm_forms import F16_SHAPES
 from gpu_util import assert_same, dev, empty, host, ptr, say, stream
 
 pytestmark = pytest.mark.gpu
@@ -405,6 +406,11 @@ F16_FORMS = [
     (16449, 200, 100, 0),                                                    # 128 x 128
     (32897, 264, 100, 0), (32897, 77, 100, 0),                               # 256 x 128
 ]
+
+
+# (then each form with stages enough to refill released slots of its ring with
+# live data, test_launch_plan.py checks which form each takes)
+F16_FORMS += [(M, K, N, 0) for _, M, K, N in F16_SHAPES]
 
 
 @pytest.mark.parametrize("M,K,N,off", F16_FORMS)

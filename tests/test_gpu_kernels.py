@@ -269,8 +269,9 @@ def test_gemm_short_k(orc, KB, form):
 @pytest.mark.parametrize("M,N", [(31, 65), (33, 1152), (300, 1003), (321, 1001), (700, 1003), (1400, 500)])
 @pytest.mark.parametrize("KB", [1, 3, 4, 5, 8, 11, 14])
 def test_gemm_latency_forms(orc, M, N, KB):
-    # 32 x 32, 32 x 64, 64 x 64 and 64 x 128 tiles at ragged edges, around
-    # whole and partial stages of 4 blocks; the sums are the oracle's bits
+    # 32 x 32, 32 x 64 and 64 x 64 tiles at ragged edges, around whole and
+    # partial stages of 4 blocks (at most 4, as many as the ring holds;
+    # test_gemm_tile_forms goes on from there); the sums are the oracle's bits
     K = 32 * KB
     say(f"gemm latency form: KB={KB} M={M} N={N}")
     rng = np.random.default_rng(90 + KB)

@@ -8,7 +8,7 @@ import subprocess
 import numpy as np
 import pytest
 
-from gemm_forms import LATENCY_SHAPES
+from gemm_forms import F16_SHAPES, F16_TOWER_ROWS, LATENCY_SHAPES
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "hbd-siglip2.cpp_amd", "csrc")
@@ -109,3 +109,11 @@ def test_q8_form_fills_the_cus_once(plan, n_split):
             if min(tiles.values()) <= 256:
                 assert tiles[got] <= 256, (M, N, got, tiles)
             assert _q8_form(plan, M, N, False) in ("Wide", "Small4", "Small3")
+
+
+def test_f16_shapes_take_their_form(plan):
+    shapes = [(f, M, K, N) for f, M, K, N in F16_SHAPES]
+    shapes += [(f, M, 4304, 1152) for f, M in F16_TOWER_ROWS.items()]
+    for form, M, K, N in shapes:
+        got = plan.plan_f16_form(ctypes.c_int64(M), ctypes.c_int64(N), ctypes.c_int64(_up(K, 64)))
+        assert ["Small", "Mid", "Wide"][got] == form, (M, K, N)
