@@ -37,21 +37,24 @@ inline bool f16_ld_ok(int64_t ld) { return 128 * ld * 2 <= 0x7fffffff; }
 
 // Operand layouts of one F16 product from raw weight rows (K halves apart)
 // and a workspace of round_up(N K_pad 2, 256) + round_up(M K_pad 2, 256)
-// bytes.  Weight rows that are 16-byte aligned (w_align16: their first one
-// is) are read in place; X then has the whole workspace for rows of whole
-// 128-byte lines, if those fit there and the GEMM takes the stride.
+// bytes.  Weight rows that are 16-byte aligned are read in place where y does
+// not lie over them (f16_w_in_place); X then has the whole workspace for rows
+// of whole 128-byte lines, if those fit there and the GEMM takes the stride.
+inline bool f16_w_in_place(uintptr_t w, uintptr_t y, int64_t K, int64_t N, int64_t M) {
+    return K % 8 == 0 && w % 16 == 0 && (y + (uintptr_t)(M * N * 4) <= w || w + (uintptr_t)(N * K * 2) <= y);
+}
 struct F16MulMatPlan {
     bool    w_direct;
     int64_t ldx16, ldw;  // halves
     int64_t x_off;       // bytes
     int64_t total;       // of the workspace
 };
-inline F16MulMatPlan f16_mul_mat_plan(int64_t K, int64_t N, int64_t M, bool w_align16) {
+inline F16MulMatPlan f16_mul_mat_plan(int64_t K, int64_t N, int64_t M, bool w_in_place) {
     const int64_t K_pad = (K + 31) / 32 * 32, ld_line = (K + 63) / 64 * 64;
     F16MulMatPlan p;
     p.x_off = (N * K_pad * 2 + 255) / 256 * 256;
     p.total = p.x_off + (M * K_pad * 2 + 255) / 256 * 256;
-    p.w_direct = K % 8 == 0 && w_align16;
+    p.w_direct = w_in_place;
     p.ldw = p.w_direct ? K : K_pad;
     p.ldx16 = K_pad;
     if (p.w_direct && M * ld_line * 2 <= p.total && f16_ld_ok(ld_line)) {

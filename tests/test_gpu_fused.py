@@ -469,6 +469,26 @@ def test_mul_mat_f16_longest_rows(K):
     assert_same(host(y), ref.float().cpu().numpy(), f"K={K}")
 
 
+@pytest.mark.parametrize("M,K,N", [(40, 64, 70), (300, 264, 130)])
+def test_mul_mat_f16_result_over_its_weight(M, K, N):
+    # y may lie over w_raw: the weight is copied before the result is written
+    say(f"F16 mul_mat y over w M={M} K={K} N={N}")
+    rng = np.random.default_rng(60)
+    w16 = rng.standard_normal((N, K)).astype(np.float16)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    xd, wsb = dev(x), s2x.lib.s2x_mul_mat_f16_workspace_size(K, N, M)
+    ws, ref = empty((wsb,), torch.uint8), None
+    for over in (False, True):
+        buf = torch.zeros(max(M * N, N * K), dtype=torch.float32, device="cuda:0")
+        buf[:N * K // 2] = dev(w16.reshape(-1).view(np.float32))
+        y = buf if over else empty((M * N,), torch.float32)
+        s2x.call("s2x_mul_mat_f16_f32", ptr(buf), K, N, ptr(xd), K, M, ptr(y), ptr(ws), ctypes.c_size_t(wsb),
+                 stream())
+        got = host(y)[:M * N]
+        ref = got if ref is None else ref
+        assert_same(got, ref, f"y over w: {over}")
+
+
 def test_mul_mat_f16_many_rows():
     # more rows than one wave each allows a launch (2^32 threads)
     M, K, N = (1 << 26) + 3, 8, 1

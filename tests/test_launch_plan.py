@@ -58,10 +58,28 @@ def test_f16_operand_grid_takes_rows_up_to_the_launch_limit(plan):
             assert _operand_grid(plan, rows, ld)[2] * 256 < 1 << 32, (K, ld, rows)
 
 
+def _w_in_place(plan, w, y, K, N, M):
+    return bool(plan.plan_f16_w_in_place(*(ctypes.c_uint64(v) for v in (w, y)),
+                                         *(ctypes.c_int64(v) for v in (K, N, M))))
+
+
 def _f16_plan(plan, K, N, M, w_align16):
     out = (ctypes.c_int64 * 5)()
-    plan.plan_f16_mul_mat(*(ctypes.c_int64(v) for v in (K, N, M)), int(w_align16), out)
+    in_place = w_align16 and _w_in_place(plan, 1 << 20, 1 << 50, K, N, M)
+    plan.plan_f16_mul_mat(*(ctypes.c_int64(v) for v in (K, N, M)), int(in_place), out)
     return tuple(out)
+
+
+def test_f16_weight_is_read_in_place_only_beside_y(plan):
+    K, N, M, w = 64, 10, 7, 1 << 20
+    end, size = w + N * K * 2, M * N * 4
+    assert _w_in_place(plan, w, end, K, N, M) and _w_in_place(plan, w, w - size, K, N, M)
+    # y over the weight, from its first byte to its last: the rows are copied
+    # first, as the result overwrites them
+    for y in (w, w + 4, end - 4, w - size + 4, w - 4):
+        assert not _w_in_place(plan, w, y, K, N, M), y - w
+    assert not _w_in_place(plan, w + 8, end + 8, K, N, M)   # alignment
+    assert not _w_in_place(plan, w, end + 4096, 63, N, M)   # of every row
 
 
 def test_f16_mul_mat_layouts_fit_the_workspace_and_the_gemm(plan):
