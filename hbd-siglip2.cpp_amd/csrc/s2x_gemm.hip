@@ -292,7 +292,7 @@ __device__ __forceinline__ void epilogue(float (&acc)[TM][TN][16], float scale, 
                                                  : (_Float16)0.0f;
                     }
             };
-            // (of a few rows only those: at M = 1 all 32 take 1.9 us longer)
+            // (of a few rows only those: M = 1, K = 96 4.6 us, with all 32 6.7)
             if (rows >= 32)
                 gelu_rows(std::true_type{});
             else
@@ -623,9 +623,9 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
     // kpos(g) = KB - KS, so its block kb0 + j lands in slot j + shift of the
     // stage buffer (shift = kb0 - kpos); a GEMM of fewer than KS blocks has
     // one partial stage, fetched by the first issue (outside the K loop)
-    // with out-of-range lanes for the missing blocks and scales.  ROLE (a constant per wave: 1 X scales, 2 W
-    // scales, 3 both, 0 neither) is a template value, so that no branch splits the
-    // K loop.
+    // with out-of-range lanes for the missing blocks and scales.  ROLE (a
+    // constant per wave: 1 X scales, 2 W scales, 3 both, 0 neither) is a
+    // template value, so that no branch splits the K loop.
     // PART: 0 the X quants, 1 the W quants, 2 the scales, -1 all three
     auto kpos = [&](int g) { return KB >= KS ? min(g * KS, KB - KS) : g * KS; };
     auto issue = [&](int g, auto role, auto part, auto first) {
@@ -1112,8 +1112,8 @@ hipError_t run(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_
 // F16 weight x f16 activation, f32 accumulation (GGML_OP_MUL_MAT with an
 // F16 weight, as the reference's converter stores ffn_down: K = 4304 is
 // not a multiple of 32).  A stage is 64 halves (a 128-byte line) of BM
-// rows of X and BN of W, brought by LDS DMA into a ring of NS stages, two of
-// them in flight while one is used; a fragment pair is read one step ahead
+// rows of X and BN of W, brought by LDS DMA into a ring of NS stages, up to
+// NS - 1 of them in flight while one is used; a fragment pair is read one step ahead
 // of its MFMAs, also over the stage's barrier.  A CU's LDS-DMA path (about
 // 64 bytes a cycle) and its matrix pipes bound it alike: 128 x 128 tiles
 // need 32 KB per 512 matrix cycles.  Its instructions therefore go between
@@ -1121,9 +1121,10 @@ hipError_t run(const WeightView &w, const int8_t *xq, int64_t ldx, const uint32_
 // the wave, and its matrix pipe, for about as long as the MFMAs take (M =
 // 2,916, K = 4,304, N = 1,152: 40.0 us, spread 37.9).  Before, with a ring of
 // two half-line stages and no fragment ahead, that product with its operand
-// conversions took 83.6 us, now 53.9; X in rows of whole lines and the raw W
-// read in place where it is aligned are part of it (W in whole lines, as the
-// towers hold it: 33.9 us).
+// conversions took 81 to 84 us, now 50 (repeated on the same buffers) to 61
+// (weights from HBM); X in rows of whole lines and the raw W read in place
+// where it is aligned are part of it (W in whole lines, as the towers hold it:
+// 33.9 us for the GEMM).
 // ---------------------------------------------------------------------------
 // BM x BN tiles of WM x WN waves, each 32 TM x 32 TN outputs; stages of 64
 // halves (128 bytes a row) in a ring of NS.
