@@ -203,8 +203,12 @@ struct Frag {
 // The GELU -> Q8_1 / f16 and QKV epilogues take 32 x 64 blocks (TN = 2).
 // The product is acc * scale (a power of two: exact), so that mm + bias is
 // one fmaf(acc, scale, bias), the same bits as (acc * scale) + bias.
+// FEW (the latency form's): a half of fewer than 32 rows of the GELU -> f16
+// epilogue computes the GELU of its rows' groups of 8 only (M = 1, K = 96
+// 6.6 us -> 4.5).  Large GEMMs have one such half per column tile and do
+// without the second path.
 constexpr int EPI_SCRATCH = 5120;
-template <int TM, int TN, int EPI>
+template <int TM, int TN, int EPI, bool FEW = false>
 __device__ __forceinline__ void epilogue(float (&acc)[TM][TN][16], float scale, const float (&bias_v)[TN], int lane,
                                          int mw, int nw, int M, int N, float *__restrict__ y,
                                          int64_t ldy, const EpiParams &epi, uint8_t *wscr) {
@@ -280,28 +284,32 @@ __device__ __forceinline__ void epilogue(float (&acc)[TM][TN][16], float scale, 
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
             const int rows = M - mw - a * 32;  // wave-uniform
-            auto gelu_rows = [&](auto whole) {
+            // rows 8 q .. 8 q + 7; columns past N as a mask, not a choice: that
+            // becomes a branch around every element's GELU
+            auto gelu_rows = [&](int b, int q) {
+                const uint32_t live = nw + b * 32 + lr < N ? ~0u : 0u;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = gelu_tanh(fmaf(acc[a][b][4 * q + r], scale, bias_v[b]));
+                    scr[(8 * q + 4 * lh + r) * P + b * 32 + lr] =
+                        f32_to_f16(__builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & live));
+                }
+            };
+            if (FEW && rows < 32) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (8 * q < rows) gelu_rows(0, q), gelu_rows(1, q);
+            } else {
 #pragma unroll
                 for (int b = 0; b < 2; ++b)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int r0 = 8 * (r >> 2) + (r & 3);  // rows r0 (lanes 0..31) and r0 + 4
-                        if (!decltype(whole)::value && r0 >= rows) continue;
-                        scr[(r0 + 4 * lh) * P + b * 32 + lr] =
-                            nw + b * 32 + lr < N ? f32_to_f16(gelu_tanh(fmaf(acc[a][b][r], scale, bias_v[b])))
-                                                 : (_Float16)0.0f;
-                    }
-            };
-            // (of a few rows only those: M = 1, K = 96 4.6 us, with all 32 6.7)
-            if (rows >= 32)
-                gelu_rows(std::true_type{});
-            else
-                gelu_rows(std::false_type{});
+                    for (int q = 0; q < 4; ++q) gelu_rows(b, q);
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int id = lane + 64 * i, row = id >> 3, c = (id & 7) * 8;
                 const int m = mw + a * 32 + row, n = nw + c;
-                if (row >= rows || n >= epi.h_kpad) continue;  // (h_kpad is a multiple of 32: whole chunks)
+                if (m >= M || n >= epi.h_kpad) continue;  // (h_kpad is a multiple of 32: whole chunks)
                 _Float16 *dst = epi.h_out + (int64_t)m * epi.h_ld + n;
                 const v8h v = *reinterpret_cast<const v8h *>(scr + row * P + c);
                 if (vec) {
@@ -1077,7 +1085,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(C::WPE)))
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
     // acc = acc' * 2^26 (exact), folded into the epilogue's first operation
-    epilogue<TM, TN, EPI>(acc, 67108864.0f, bias_v, lane, m0 + wm * 32 * TM, n0 + wn * 32 * TN, M, N, y, ldy, epi,
+    epilogue<TM, TN, EPI, C::LAT>(acc, 67108864.0f, bias_v, lane, m0 + wm * 32 * TM, n0 + wn * 32 * TN, M, N, y, ldy, epi,
                       lds + wave * EPI_SCRATCH);
     // Every DMA this wave issued has landed before the workgroup ends.
     wait_vm<0>();
