@@ -59,8 +59,9 @@
 // lines apart), not 32 bytes of 32 rows: the vector memory path handles an
 // instruction line by line (1 KB as 8 whole lines takes it 15 to 17 cycles,
 // as 32 quarter lines 30, measured alone).  It is what the few-rows forms
-// wait for: M = 729 fc2 23.3 -> 20.8 us, M = 64 fc2 21.6 -> 17.7; at M =
-// 23,328, where the matrix pipe and the VALU bound the loop, 1 to 3 %.
+// wait for: M = 729 fc2 23.3 -> 20.8 us, M = 64 fc2 21.6 -> 17.7; a step of
+// 23,328 rows, where the matrix pipe and the VALU bound the loop, gains 1 to
+// 1.5 %, about what runs differ.
 #include "s2x_device.h"
 #include "s2x_kernels.h"
 #include "s2x_plan.h"

@@ -440,7 +440,8 @@ int s2x_vision_set_graphs(s2x_vision *v, int enable);
  * the default path meets.
  * 1 = the vision tower's plain and residual GEMMs of 32+ K blocks (out,
  * fc2, the head's) run as s2x_mul_mat_q8_0_q8_1_split_k (2 ranges, 4 from
- * 96 blocks), for latency at batch 1; 0 (default) = one block-order sum per
+ * 96 blocks), once for latency at batch 1 (3.09 ms, where the default's forms
+ * for few rows now take 2.75); 0 (default) = one block-order sum per
  * output, the oracle's.  No counterpart in the reference (whose GPU GEMMs
  * split K by stream-K); an image's bits do not depend on its batch either
  * way.  Batch 32 runs slower with it (partial sums of 4 x 107 MB per fc2). */
@@ -502,8 +503,9 @@ int s2x_text_set_graphs(s2x_text *t, int enable);
 /* EXPERIMENTAL, outside the parity tolerance (cosine 0.99988 of the
  * block-order CPU restatement on the so400m text tower, below 0.9999).
  * 1 = the text tower's plain and residual GEMMs of 32+ K blocks run as
- * s2x_mul_mat_q8_0_q8_1_split_k (2 ranges, 4 from 96 blocks); 0 (default) =
- * one block-order sum per output, the oracle's.  No counterpart in the
+ * s2x_mul_mat_q8_0_q8_1_split_k (2 ranges, 4 from 96 blocks: 2.44 ms for 5 x
+ * 64 tokens, the default 2.30); 0 (default) = one block-order sum per output,
+ * the oracle's.  No counterpart in the
  * reference (whose GPU GEMMs split K by stream-K); a prompt's bits do not
  * depend on its batch either way. */
 int s2x_text_set_split_k(s2x_text *t, int enable);
