@@ -274,7 +274,7 @@ int s2x_mul_mat_q8_0_f32(const void *w_raw, int64_t K_pad, int64_t N, const floa
 
 size_t s2x_mul_mat_f16_workspace_size(int64_t K, int64_t N, int64_t M) {
     if (K <= 0 || N <= 0 || M < 0) return 0;
-    return (size_t)f16_mul_mat_plan(K, N, M, false).total;
+    return (size_t)f16_mul_mat_ws_bytes(K, N, M);
 }
 
 int s2x_mul_mat_f16_f32(const void *w_raw, int64_t K, int64_t N, const float *x, int64_t ldx,
@@ -287,7 +287,8 @@ int s2x_mul_mat_f16_f32(const void *w_raw, int64_t K, int64_t N, const float *x,
         return fail(S2X_ERR_UNSUPPORTED, "mul_mat_f16_f32: shape too large");
     if (!w_raw || !x || !y || !workspace)
         return fail(S2X_ERR_INVALID_ARG, "mul_mat_f16_f32: null pointer");
-    const F16MulMatPlan L = f16_mul_mat_plan(K, N, M, f16_w_in_place((uintptr_t)w_raw, (uintptr_t)y, K, N, M));
+    const F16MulMatPlan L = f16_mul_mat_plan(
+        K, N, M, f16_w_in_place((uintptr_t)w_raw, (uintptr_t)y, (uintptr_t)workspace, K, N, M));
     if (ws_bytes < (size_t)L.total)
         return fail(S2X_ERR_WORKSPACE, "mul_mat_f16_f32: workspace %zu < %zu bytes", ws_bytes, (size_t)L.total);
     if (!aligned(workspace, 256) || !aligned(w_raw, 2) || !aligned(x, 4) || !aligned(y, 4))

@@ -37,12 +37,10 @@ inline bool f16_ld_ok(int64_t ld) { return 128 * ld * 2 <= 0x7fffffff; }
 
 // Operand layouts of one F16 product from raw weight rows (K halves apart)
 // and a workspace of round_up(N K_pad 2, 256) + round_up(M K_pad 2, 256)
-// bytes.  Weight rows that are 16-byte aligned are read in place where y does
-// not lie over them (f16_w_in_place); X then has the whole workspace for rows
-// of whole 128-byte lines, if those fit there and the GEMM takes the stride.
-inline bool f16_w_in_place(uintptr_t w, uintptr_t y, int64_t K, int64_t N, int64_t M) {
-    return K % 8 == 0 && w % 16 == 0 && (y + (uintptr_t)(M * N * 4) <= w || w + (uintptr_t)(N * K * 2) <= y);
-}
+// bytes.  Weight rows that are 16-byte aligned are read in place where neither
+// y nor the workspace lies over them (f16_w_in_place); X then has the whole
+// workspace for rows of whole 128-byte lines, if those fit there and the GEMM
+// takes the stride.
 struct F16MulMatPlan {
     bool    w_direct;
     int64_t ldx16, ldw;  // halves
@@ -62,6 +60,14 @@ inline F16MulMatPlan f16_mul_mat_plan(int64_t K, int64_t N, int64_t M, bool w_in
         p.x_off = 0;
     }
     return p;
+}
+
+inline int64_t f16_mul_mat_ws_bytes(int64_t K, int64_t N, int64_t M) { return f16_mul_mat_plan(K, N, M, false).total; }
+inline bool f16_w_in_place(uintptr_t w, uintptr_t y, uintptr_t ws, int64_t K, int64_t N, int64_t M) {
+    const auto apart = [&](uintptr_t p, int64_t bytes) {
+        return p + (uintptr_t)bytes <= w || w + (uintptr_t)(N * K * 2) <= p;
+    };
+    return K % 8 == 0 && w % 16 == 0 && apart(y, M * N * 4) && apart(ws, f16_mul_mat_ws_bytes(K, N, M));
 }
 
 // The tile form of an F16 product, by tiles per round of the 256 CUs (every

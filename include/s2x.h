@@ -152,8 +152,8 @@ int s2x_mul_mat_q8_0_f32(const void *w_raw, int64_t K_pad, int64_t N,
  * gguf.py:241-290, kept F16 by src/siglip2_vision.cpp:496-556).  X is
  * rounded to f16 (as ggml converts the F32 operand of an F16 dot) and the
  * products accumulate in f32 on f16 MFMA.  w_raw: N rows of K halves on the
- * device.  Where K is a multiple of 8, w_raw 16-byte aligned and y elsewhere, the
- * GEMM reads w_raw in place; otherwise its rows are first copied, zero-padded
+ * device.  Where K is a multiple of 8, w_raw 16-byte aligned and y and the
+ * workspace elsewhere, the GEMM reads w_raw in place; otherwise its rows are first copied, zero-padded
  * to a multiple of 32 halves, into `workspace`, as X's always are
  * (s2x_mul_mat_f16_workspace_size() bytes, 256-byte aligned).  Either way
  * w_raw stays valid and unchanged until the call's work on `stream` has

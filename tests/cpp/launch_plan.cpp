@@ -6,8 +6,8 @@ void plan_f16_operand_grid(int64_t rows, int64_t ld, int64_t *out) {
     const s2x::F16OperandGrid g = s2x::f16_operand_grid(rows, ld);
     out[0] = g.lg_lanes, out[1] = g.col_blocks, out[2] = g.blocks;
 }
-int plan_f16_w_in_place(uintptr_t w, uintptr_t y, int64_t K, int64_t N, int64_t M) {
-    return s2x::f16_w_in_place(w, y, K, N, M);
+int plan_f16_w_in_place(uintptr_t w, uintptr_t y, uintptr_t ws, int64_t K, int64_t N, int64_t M) {
+    return s2x::f16_w_in_place(w, y, ws, K, N, M);
 }
 void plan_f16_mul_mat(int64_t K, int64_t N, int64_t M, int w_in_place, int64_t *out) {
     const s2x::F16MulMatPlan p = s2x::f16_mul_mat_plan(K, N, M, w_in_place != 0);

@@ -471,17 +471,22 @@ def test_mul_mat_f16_longest_rows(K):
 
 @pytest.mark.parametrize("M,K,N", [(40, 64, 70), (300, 264, 130)])
 def test_mul_mat_f16_result_over_its_weight(M, K, N):
-    # y may lie over w_raw: the weight is copied before the result is written
+    # y may lie over w_raw: the weight is copied before the result is written.
+    # So may the front of the workspace where the copy is the weight itself
+    # (K % 32 == 0)
     say(f"F16 mul_mat y over w M={M} K={K} N={N}")
     rng = np.random.default_rng(60)
     w16 = rng.standard_normal((N, K)).astype(np.float16)
     x = rng.standard_normal((M, K)).astype(np.float32)
     xd, wsb = dev(x), s2x.lib.s2x_mul_mat_f16_workspace_size(K, N, M)
     ws, ref = empty((wsb,), torch.uint8), None
-    for over in (False, True):
-        buf = torch.zeros(max(M * N, N * K), dtype=torch.float32, device="cuda:0")
+    for over in (False, True, "ws"):
+        if over == "ws" and K % 32:
+            continue
+        buf = torch.zeros(max(M * N, N * K, wsb // 4), dtype=torch.float32, device="cuda:0")
         buf[:N * K // 2] = dev(w16.reshape(-1).view(np.float32))
-        y = buf if over else empty((M * N,), torch.float32)
+        y = buf if over is True else empty((M * N,), torch.float32)
+        ws = buf if over == "ws" else ws
         s2x.call("s2x_mul_mat_f16_f32", ptr(buf), K, N, ptr(xd), K, M, ptr(y), ptr(ws), ctypes.c_size_t(wsb),
                  stream())
         got = host(y)[:M * N]

@@ -58,8 +58,8 @@ def test_f16_operand_grid_takes_rows_up_to_the_launch_limit(plan):
             assert _operand_grid(plan, rows, ld)[2] * 256 < 1 << 32, (K, ld, rows)
 
 
-def _w_in_place(plan, w, y, K, N, M):
-    return bool(plan.plan_f16_w_in_place(*(ctypes.c_uint64(v) for v in (w, y)),
+def _w_in_place(plan, w, y, K, N, M, ws=1 << 51):
+    return bool(plan.plan_f16_w_in_place(*(ctypes.c_uint64(v) for v in (w, y, ws)),
                                          *(ctypes.c_int64(v) for v in (K, N, M))))
 
 
@@ -78,6 +78,12 @@ def test_f16_weight_is_read_in_place_only_beside_y(plan):
     # first, as the result overwrites them
     for y in (w, w + 4, end - 4, w - size + 4, w - 4):
         assert not _w_in_place(plan, w, y, K, N, M), y - w
+    # the same for the workspace, where X's rows are written first (a weight
+    # with K % 32 == 0 may lie where its own copy goes, at the front of it)
+    far, total = 1 << 50, _f16_plan(plan, K, N, M, False)[4]
+    assert _w_in_place(plan, w, far, K, N, M, end) and _w_in_place(plan, w, far, K, N, M, w - total)
+    for ws in (w, w + 256, w - 256, w - total + 256):
+        assert not _w_in_place(plan, w, far, K, N, M, ws), ws - w
     assert not _w_in_place(plan, w + 8, end + 8, K, N, M)   # alignment
     assert not _w_in_place(plan, w, end + 4096, 63, N, M)   # of every row
 
