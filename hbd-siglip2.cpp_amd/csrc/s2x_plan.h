@@ -100,7 +100,10 @@ enum class Q8Form {
     Small3   //   64 x 128, three stages, two workgroups per CU
 };
 // Wide for GEMMs of at least two 128 x 128 tiles per CU; below that the
-// latency form (M = 729 in 128 x 128 tiles: out 19.8 us, fc2 58.7).  The
+// latency form (M = 729 in 128 x 128 tiles: out 19.8 us, fc2 58.7).  Near that
+// line the two are within 8 % either way, by how full their last rounds are
+// (K = 4320, N = 4304: M = 1800, 510 tiles, Small3 81.7 us, Wide 76.4; M =
+// 2048, 544 tiles, 101.1 and 108.6).  The
 // epilogues that work on 32 x 64 blocks (plain false: GELU -> Q8_1 / F16, QKV)
 // have the 64 x 128 tiles, with four stages in the ring (three in flight)
 // where their workgroups fit one per CU and three stages (two per CU)
